@@ -65,7 +65,7 @@ def listed():
         # the five 5-vertex shapes on a social-network-like graph, mid-sized
         # (other labels in every set of inputs) and large (the same labels)
         _graph("shapes_100k", "shapes", 100000, 2.1, 20.0, 600.0, 16, 1.2),
-        _graph("shapes_1m", "shapes", 1000000, 2.1, 20.0, 0.0, 16, 1.2, shape_seed=0x47454E02 + 100),
+        _graph("shapes_1m", "shapes", 1000000, 2.1, 20.0, 1200.0, 16, 1.2, shape_seed=0x47454E02 + 100),
         # induced cyclic queries of 6-8 vertices on a graph with heavy hubs
         _graph("cyclic_hub_graph", "cyclic", 40000, 1.9, 30.0, 1000.0, 64, 1.0, queries=12, kmin=6, kmax=8),
         # walk queries on one large graph, all in one call
