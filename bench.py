@@ -235,6 +235,54 @@ def pmc_table(path):
 # workload 3 (headline): batched engine vs plain path
 
 
+def slots_roofline(eng, qs):
+    """Accounting run of the slot engine: every kernel of the iteration
+    launched on its own under HIP events, and the bytes B charged to k_b_size /
+    k_b_walk."""
+    eng.batch_profile(True)
+    eng.profile(True, count_bytes=False)
+    acct_res, acct_st = eng.mine_batch(qs)
+    prof = eng.profile_read()
+    b_size, b_walk = eng.batch_profile_bytes()
+    eng.profile(False)
+    eng.batch_profile(False)
+    kinds = {"k_b_size": prof["k_size"], "k_b_scan": prof["k_scan"], "k_b_walk": prof["k_walk<extend>"],
+             "k_b_prep/tiles/post": prof["batch_iteration"]}
+    b_total = sum(r.alg_bytes for r in acct_res)
+    dev_ms = sum(v[1] for v in kinds.values())
+    tpath = os.path.join(ROOT, "profiles", "traffic_workload3.json")
+    tjs = json.load(open(tpath)) if os.path.exists(tpath) else {}
+
+    def kernel_roofline(name, b_bytes, charged):
+        launches, ms = kinds[name][0], kinds[name][1]
+        avg_ms = ms / max(launches, 1)
+        b_launch = b_bytes // max(launches, 1)
+        achieved = b_launch / (avg_ms / 1e3) / 1e9 if avg_ms > 0 else 0.0
+        return {"bound": "hbm", "kernel": name, "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
+                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+                "traffic": tjs.get(name, {}).get("hbm_bytes_per_launch"),
+                "launches": launches, "avg_launch_ms": round(avg_ms, 4), "total_ms": round(ms, 3),
+                "b_bytes_per_launch": b_launch, "b_charged": charged}
+
+    rs = [kernel_roofline("k_b_size", b_size, "each row's read (4L), each required list (8 + 4|N|) and the "
+                                              "B of the rows it counts itself (count modes, leaf groups)"),
+          kernel_roofline("k_b_walk", b_walk, "the survivors' writes (4(L+1) each) and, in a counted step, "
+                                              "the lists its fused last vertex searches")]
+    # the dominant kernel (most device time per step) is the line's roofline;
+    # the other is reported beside it
+    rs.sort(key=lambda r: -r["total_ms"])
+    roofline = dict(rs[0])
+    roofline["other"] = rs[1]
+    # B the kernels executed (k_b_size + k_b_walk) over the whole iteration's
+    # device time; the queries' own B also counts the steps shared between
+    # queries once per query and the closed-form first steps of pair starts
+    roofline["iteration"] = {"b_bytes": b_size + b_walk, "device_ms": round(dev_ms, 3),
+                             "frac": round((b_size + b_walk) / (max(dev_ms, 1e-9) / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
+                             "b_bytes_of_queries": b_total}
+    kern = {k: {"launches": v[0], "ms": round(v[1], 3)} for k, v in kinds.items()}
+    return roofline, kern
+
+
 def section_w3(args):
     import numpy as np  # noqa: F401
     import geneva_amd as G
@@ -280,50 +328,25 @@ def section_w3(args):
               for q, r in zip(qs, batched)]
         parity.update({"checked": len(ok), "bit_exact": sum(ok),
                        "against": "oracle fixture tests/golden/workload3_full.json (counts, bytes, graph-id sets)"})
-    # one accounting run: every kernel of the iteration launched on its own
-    # under HIP events, and the bytes B charged to k_b_size / k_b_walk
     shared = dict(zip(("shared", "restarted"), eng.batch_share_stats()))
-    eng.batch_profile(True)
+    # one accounting run out of the packed database: its mining launches under
+    # HIP events, and the bytes B of the steps they ran
     eng.profile(True, count_bytes=False)
     acct_res, acct_st = eng.mine_batch(qs)
-    prof = eng.profile_read()
-    b_size, b_walk = eng.batch_profile_bytes()
+    launches, dev_ms, _, _, b_ran = eng.profile_read()["k_resident"]
     eng.profile(False)
-    eng.batch_profile(False)
-    kinds = {"k_b_size": prof["k_size"], "k_b_scan": prof["k_scan"], "k_b_walk": prof["k_walk<extend>"],
-             "k_b_prep/tiles/post": prof["batch_iteration"]}
     b_total = sum(r.alg_bytes for r in acct_res)
-    dev_ms = sum(v[1] for v in kinds.values())
-    tpath = os.path.join(ROOT, "profiles", "traffic_workload3.json")
-    tjs = json.load(open(tpath)) if os.path.exists(tpath) else {}
-
-    def kernel_roofline(name, b_bytes, charged):
-        launches, ms = kinds[name][0], kinds[name][1]
-        avg_ms = ms / max(launches, 1)
-        b_launch = b_bytes // max(launches, 1)
-        achieved = b_launch / (avg_ms / 1e3) / 1e9 if avg_ms > 0 else 0.0
-        return {"bound": "hbm", "kernel": name, "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": tjs.get(name, {}).get("hbm_bytes_per_launch"),
-                "launches": launches, "avg_launch_ms": round(avg_ms, 4), "total_ms": round(ms, 3),
-                "b_bytes_per_launch": b_launch, "b_charged": charged}
-
-    rs = [kernel_roofline("k_b_size", b_size, "each row's read (4L), each required list (8 + 4|N|) and the "
-                                              "B of the rows it counts itself (count modes, leaf groups)"),
-          kernel_roofline("k_b_walk", b_walk, "the survivors' writes (4(L+1) each) and, in a counted step, "
-                                              "the lists its fused last vertex searches")]
-    # the dominant kernel (most device time per step) is the line's roofline;
-    # the other is reported beside it
-    rs.sort(key=lambda r: -r["total_ms"])
-    roofline = dict(rs[0])
-    roofline["other"] = rs[1]
-    # B the kernels executed (k_b_size + k_b_walk) over the whole iteration's
-    # device time; the queries' own B also counts the steps shared between
-    # queries once per query and the closed-form first steps of pair starts
-    roofline["iteration"] = {"b_bytes": b_size + b_walk, "device_ms": round(dev_ms, 3),
-                             "frac": round((b_size + b_walk) / (max(dev_ms, 1e-9) / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
-                             "b_bytes_of_queries": b_total}
-    kern = {k: {"launches": v[0], "ms": round(v[1], 3)} for k, v in kinds.items()}
+    if launches:
+        achieved = b_ran / (dev_ms / 1e3) / 1e9 if dev_ms > 0 else 0.0
+        roofline = {"bound": "lds", "kernel": "k_resident", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
+                    "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "launches": launches,
+                    "avg_launch_ms": round(dev_ms / launches, 4), "total_ms": round(dev_ms, 3),
+                    "b_bytes_per_launch": b_ran // launches, "b_bytes_of_queries": b_total,
+                    "b_charged": "B of every step run, steps shared between queries once; the kernel reads it out "
+                                 "of LDS, so HBM's rate is a scale here and no limit"}
+        kern = {"k_resident": {"launches": launches, "ms": round(dev_ms, 3)}}
+    else:
+        roofline, kern = slots_roofline(eng, qs)
     out = {"embeddings_per_step": emb, "queries": len(qs), "ms_per_step": ms_step,
            "batched_queries_per_s": round(len(qs) / (ms_step / 1e3), 1),
            "plain_ms": round(tp, 3), "plain_queries_per_s": round(len(qs) / (tp / 1e3), 1),

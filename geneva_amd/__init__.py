@@ -351,7 +351,7 @@ class Engine:
 
     KERNELS = {0: "k_size", 1: "k_scan", 2: "k_walk<extend>", 3: "k_walk<count>",
                4: "batch_iteration", 5: "k_count_rows", 6: "k_isect", 7: "k_count_chain",
-               8: "ref_launchers"}
+               8: "ref_launchers", 9: "k_resident"}
 
     def batch_config(self, slots=0, slot_bytes=0, row_cap=0, ipt=0, blocks_per_cu=0):
         """Configure the batch engine (0 keeps a setting); rebuilt on next use."""

@@ -1101,11 +1101,14 @@ bool tune_ok(const gv_tune_t* t) {
 
 extern "C" {
 
+int gv_batch_check(uint32_t slots, uint64_t slot_bytes, uint64_t row_cap, const gv_tune_t* tune) {
+    if (slots == 0 || slots > kMaxSlots || slot_bytes < 4096 || row_cap == 0) return GV_ERR_ARG;
+    return tune && !tune_ok(tune) ? GV_ERR_ARG : GV_OK;
+}
+
 int gv_batch_create(gv_ctx_t c, gv_graph_t g, uint32_t slots, uint64_t slot_bytes,
                     uint64_t row_cap, const gv_tune_t* tune, gv_batch_t* out) {
-    if (!c || !g || !out || slots == 0 || slots > kMaxSlots || slot_bytes < 4096 || row_cap == 0)
-        return GV_ERR_ARG;
-    if (tune && !tune_ok(tune)) return GV_ERR_ARG;
+    if (!c || !g || !out || gv_batch_check(slots, slot_bytes, row_cap, tune) != GV_OK) return GV_ERR_ARG;
     // a sizing tile's candidate prefix is kept in 32 bits
     if ((uint64_t)g->max_deg * kBSizeTile >= (1ull << 32)) return GV_ERR_ARG;
     *out = nullptr;

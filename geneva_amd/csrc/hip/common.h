@@ -1192,10 +1192,15 @@ struct gv_ctx {
     // workspace and resume state of the reference-layout launchers
     // (launchers.hip), created on their first call
     struct RefState* ref = nullptr;
+    // buffers of gv_resident_mine (resident.hip), created on its first call
+    struct ResWork* resw = nullptr;
+    uint64_t res_bytes = 0;   // algorithmic bytes of its profiled launches
 };
 
 // Frees ctx->ref (launchers.hip); called by gv_ctx_destroy.
 void ref_state_free(gv_ctx* c);
+// Frees ctx->resw (resident.hip); called by gv_ctx_destroy.
+void res_work_free(gv_ctx* c);
 
 struct gv_graph {
     gv_ctx* ctx = nullptr;
@@ -1222,7 +1227,13 @@ struct gv_graph {
     std::vector<uint64_t> pe_off, pel_off;
     uint32_t* d_pe = nullptr;
     uint32_t* d_pel = nullptr;
+    // a database packed graph by graph (resident.hip); null when it cannot be
+    struct ResImage* res = nullptr;
 };
+
+// Pack a graph that has its owners (resident.hip), and free the packed form.
+int res_image_build(gv_graph* g, const uint32_t* graph_of);
+void res_image_free(gv_graph* g);
 
 struct gv_frontier {
     gv_ctx* ctx = nullptr;
@@ -1251,7 +1262,7 @@ DevGraph dev_view(const gv_graph* g) {
 }
 
 enum { kKindSize = 0, kKindScan = 1, kKindExt = 2, kKindCount = 3, kKindBatch = 4, kKindRows = 5,
-       kKindIsect = 6, kKindChain = 7, kKindRef = 8, kKinds = 9 };
+       kKindIsect = 6, kKindChain = 7, kKindRef = 8, kKindResident = 9, kKinds = 10 };
 
 hipEvent_t pool_get(gv_ctx* c) {
     if (!c->pool.empty()) {

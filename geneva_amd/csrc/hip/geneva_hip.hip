@@ -1095,6 +1095,7 @@ int gv_ctx_destroy(gv_ctx_t c) {
     if (c->pmark) hipFree(c->pmark);
     if (c->plist) hipFree(c->plist);
     ref_state_free(c);
+    res_work_free(c);
     for (auto& r : c->recs) {
         hipEventDestroy(r.a);
         hipEventDestroy(r.b);
@@ -1351,6 +1352,7 @@ int gv_graph_destroy(gv_graph_t g) {
     if (g->d_pe) hipFree(g->d_pe);
     if (g->d_pel) hipFree(g->d_pel);
     if (g->d_gof) hipFree(g->d_gof);
+    res_image_free(g);
     delete g;
     return GV_OK;
 }
@@ -1364,7 +1366,12 @@ int gv_graph_set_owner(gv_graph_t g, const uint32_t* graph_of, uint32_t ngraphs)
     if (hipMalloc(&g->d_gof, g->nv1 * sizeof(uint32_t)) != hipSuccess) return GV_ERR_NOMEM;
     HIPCHK(hipMemcpy(g->d_gof, graph_of, g->nv1 * sizeof(uint32_t), hipMemcpyHostToDevice));
     g->ngraphs = ngraphs;
-    return GV_OK;
+    const int rc = res_image_build(g, graph_of);
+    if (rc == GV_OK) return rc;
+    res_image_free(g);
+    // without the memory for it the table engines mine the database
+    if (rc == GV_ERR_NOMEM) (void)hipGetLastError();
+    return rc == GV_ERR_NOMEM ? GV_OK : rc;
 }
 
 int gv_graph_owners(gv_graph_t g, uint32_t* ngraphs) {
@@ -2132,6 +2139,7 @@ int gv_profile_reset(gv_ctx_t c) {
         c->pool.push_back(r.b);
     }
     c->recs.clear();
+    c->res_bytes = 0;
     if (c->preq) HIPCHK(hipMemsetAsync(c->preq, 0, kKinds * sizeof(unsigned long long), c->stream));
     if (c->punits) HIPCHK(hipMemsetAsync(c->punits, 0, 2 * kKinds * sizeof(unsigned long long), c->stream));
     return GV_OK;
@@ -2151,8 +2159,8 @@ int gv_profile_units(gv_ctx_t c, int kind, uint64_t* units) {
 
 int gv_profile_alg_bytes(gv_ctx_t c, int kind, uint64_t* bytes) {
     if (!c || !bytes || kind < 0 || kind >= kKinds) return GV_ERR_ARG;
-    *bytes = 0;
-    if (c->punits) {
+    *bytes = kind == kKindResident ? c->res_bytes : 0;
+    if (c->punits && kind != kKindResident) {
         unsigned long long h[2 * kKinds];
         HIPCHK(hipMemcpyAsync(h, c->punits, sizeof(h), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));

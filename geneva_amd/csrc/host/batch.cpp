@@ -58,23 +58,122 @@ BatchMiner::~BatchMiner() {
 }
 
 int BatchMiner::init() {
-    if (b_) return GV_OK;
     uint32_t ng = 0;
     gv_graph_owners(g_, &ng);
     nwords_ = (ng + 31) / 32;
-    return gv_batch_create(ctx_, g_, opt_.slots, opt_.slotBytes, opt_.rowCap, &opt_.tune, &b_);
+    uint32_t blocks = 0;
+    gv_resident_info(g_, &blocks, nullptr);
+    if (blocks) return gv_batch_check(opt_.slots, opt_.slotBytes, opt_.rowCap, &opt_.tune);
+    gv_batch_t b;
+    return engine(&b);
+}
+
+int BatchMiner::engine(gv_batch_t* b) {
+    if (!b_) {
+        int rc = gv_batch_create(ctx_, g_, opt_.slots, opt_.slotBytes, opt_.rowCap, &opt_.tune, &b_);
+        if (rc == GV_OK && !share_) rc = gv_batch_share(b_, 0);
+        if (rc == GV_OK && !pairStart_) rc = gv_batch_pair_start(b_, 0);
+        if (rc == GV_OK && !fuse_) rc = gv_batch_fuse_sizing(b_, 0);
+        if (rc == GV_OK && profile_) rc = gv_batch_profile(b_, 1);
+        if (rc == GV_OK && rowCap_) rc = gv_batch_set_row_cap(b_, rowCap_);
+        if (rc != GV_OK) {
+            if (b_) gv_batch_destroy(b_);
+            b_ = nullptr;
+            return rc;
+        }
+    }
+    *b = b_;
+    return GV_OK;
 }
 
 int BatchMiner::setRowCap(uint64_t rows) {
-    int rc = gv_batch_set_row_cap(b_, rows);
+    gv_batch_t b;
+    int rc = engine(&b);
+    if (rc == GV_OK) rc = gv_batch_set_row_cap(b, rows);
     if (rc == GV_OK) rowCap_ = rows;
     return rc;
 }
 
 int BatchMiner::setTune(const gv_tune_t& t) {
-    int rc = gv_batch_set_tune(b_, &t);
+    gv_batch_t b;
+    int rc = engine(&b);
+    if (rc == GV_OK) rc = gv_batch_set_tune(b, &t);
     if (rc == GV_OK) opt_.tune = t;
     return rc;
+}
+
+int BatchMiner::setShare(bool on) {
+    share_ = on;
+    return b_ ? gv_batch_share(b_, on) : GV_OK;
+}
+int BatchMiner::setFuse(bool on) {
+    fuse_ = on;
+    return b_ ? gv_batch_fuse_sizing(b_, on) : GV_OK;
+}
+int BatchMiner::setPairStart(bool on) {
+    pairStart_ = on;
+    return b_ ? gv_batch_pair_start(b_, on) : GV_OK;
+}
+int BatchMiner::setProfile(bool on) {
+    profile_ = on;
+    gv_batch_t b;
+    int rc = engine(&b);
+    return rc == GV_OK ? gv_batch_profile(b, on) : rc;
+}
+int BatchMiner::shareStats(uint64_t* shared, uint64_t* restarted) {
+    uint64_t s = 0, r = 0;
+    int rc = b_ ? gv_batch_share_stats(b_, &s, &r) : GV_OK;
+    if (shared) *shared = s + resShared_;
+    if (restarted) *restarted = r;
+    return rc;
+}
+int BatchMiner::fusedRows(uint64_t* rows) {
+    *rows = 0;
+    int rc = b_ ? gv_batch_fused_rows(b_, rows) : GV_OK;
+    *rows += resFused_;
+    return rc;
+}
+
+// The slot engine keeps the calls that ask for it: one of its switches is off its
+// default, its byte counters are on, it is being tuned, or its tables are
+// under kResidentSlotBytes, which asks for pieces of bounded size.
+constexpr uint64_t kResidentSlotBytes = 1ull << 20;
+bool BatchMiner::resident() const {
+    return gv_resident_ready(ctx_, g_) && share_ && fuse_ && pairStart_ && !profile_ && !slotsOnly_ &&
+           opt_.slotBytes >= kResidentSlotBytes;
+}
+
+int BatchMiner::runResident(const std::vector<CompiledQuery>& qs, const std::vector<size_t>& order,
+                            std::vector<MineResult>& out, BatchStats& st) {
+    const size_t n = order.size();
+    std::vector<const gv_query_t*> q(n);
+    std::vector<const gv_leaves_t*> lv(n);
+    std::vector<uint64_t> count(n), bytes(n);
+    std::vector<uint32_t*> bits(n);
+    for (size_t i = 0; i < n; ++i) {
+        const CompiledQuery& cq = qs[order[i]];
+        q[i] = &cq.q;
+        lv[i] = cq.hasLeaves ? &cq.leaves : nullptr;
+        out[order[i]].graphBits.assign(nwords_, 0);
+        bits[i] = out[order[i]].graphBits.data();
+    }
+    gv_mark(ctx_, 2);
+    int rc = gv_resident_mine(ctx_, g_, (uint32_t)n, q.data(), lv.data(), count.data(), bytes.data(),
+                              nwords_ ? bits.data() : nullptr, nwords_, &res_);
+    if (rc != GV_OK) return rc;
+    gv_mark(ctx_, 3);
+    float ms = 0;
+    gv_elapsed_ms(ctx_, 2, 3, &ms);
+    st.deviceMs = ms;
+    st.batched = n;
+    st.graphLaunches += res_.launches;
+    resShared_ += res_.shared_queries;
+    resFused_ += res_.fused_rows;
+    for (size_t i = 0; i < n; ++i) {
+        out[order[i]].count = count[i];
+        out[order[i]].algBytes = bytes[i];
+    }
+    return GV_OK;
 }
 
 std::string BatchMiner::classKey(const CompiledQuery& cq) {
@@ -117,6 +216,25 @@ int BatchMiner::run(const std::vector<CompiledQuery>& qs, std::vector<MineResult
     };
     std::stable_sort(order.begin(), order.end(),
                      [&](size_t a, size_t b) { return startKey(a) < startKey(b); });
+    BatchStats local;
+    res_ = gv_resident_stats_t{};
+    if (resident()) {
+        // the packed form takes what it can, the slot engine the others
+        std::vector<size_t> packed, rest;
+        for (size_t i : order)
+            (residentTakes(qs[i]) ? packed : rest).push_back(i);
+        rc = packed.empty() ? GV_OK : runResident(qs, packed, out, local);
+        if (rc == GV_OK) order.swap(rest);
+        else if (rc != GV_ERR_CAPACITY) return rc;
+        if (order.empty()) {
+            local.wallMs = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
+            if (st) *st = local;
+            return GV_OK;
+        }
+    }
+    gv_batch_t b = nullptr;
+    rc = engine(&b);
+    if (rc != GV_OK) return rc;
     // a query whose table outgrows its slot comes back as two pieces of its
     // first table (each piece that overflows splits again), up to kMaxPieces;
     // beyond that it is mined on the plain path
@@ -160,7 +278,6 @@ int BatchMiner::run(const std::vector<CompiledQuery>& qs, std::vector<MineResult
     std::vector<Piece> slotPiece(opt_.slots, Piece{SIZE_MAX, 0, 0});
     std::vector<gv_slot_info_t> info(opt_.slots);
     std::vector<uint32_t> bits;
-    BatchStats local;
     uint32_t running = 0;
     gv_mark(ctx_, 2);
     while (!pending.empty() || running > 0) {
@@ -241,7 +358,7 @@ int BatchMiner::run(const std::vector<CompiledQuery>& qs, std::vector<MineResult
     gv_mark(ctx_, 3);
     float ms = 0;
     gv_elapsed_ms(ctx_, 2, 3, &ms);
-    local.deviceMs = ms;
+    local.deviceMs += ms;
     const auto f0 = std::chrono::steady_clock::now();
     for (size_t qi : overflow) {
         local.overflowed++;
@@ -301,6 +418,12 @@ std::string shapeKey(const std::vector<CompiledQuery>& qs) {
 
 int autotune(BatchMiner& bm, const std::vector<CompiledQuery>& sample, TuneResult& out) {
     out = TuneResult();
+    // the settings are the slot engine's: it runs the samples
+    struct Slots {
+        BatchMiner& bm;
+        explicit Slots(BatchMiner& b) : bm(b) { bm.useSlots(true); }
+        ~Slots() { bm.useSlots(false); }
+    } slots(bm);
     const std::string key = graphKey(bm.graph(), bm.options()) + shapeKey(sample);
     {
         std::lock_guard<std::mutex> l(tuneMutex());

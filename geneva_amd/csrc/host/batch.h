@@ -50,17 +50,33 @@ public:
     BatchMiner(const BatchMiner&) = delete;
     BatchMiner& operator=(const BatchMiner&) = delete;
 
+    // Checks the options; the slot engine itself is made when it is first
+    // needed (a packed database mostly runs without it).
     int init();
+    int engine(gv_batch_t* b);
     int setTune(const gv_tune_t& t);
     // Rows sized per iteration (at most options().rowCap, the allocation).
     int setRowCap(uint64_t rows);
     uint64_t rowCap() const { return rowCap_ ? rowCap_ : opt_.rowCap; }
     const BatchOptions& options() const { return opt_; }
-    gv_batch_t handle() const { return b_; }
     gv_graph_t graph() const { return g_; }
     PlainMiner* fallback() const { return fallback_; }
     // words of a matched-graph bitset (0 without an owner table); valid after init()
     uint32_t graphWords() const { return nwords_; }
+
+    // Switches of the slot engine (gv_batch_share, gv_batch_fuse_sizing,
+    // gv_batch_pair_start, gv_batch_profile) and its counters, those of a
+    // packed database's queries included.
+    int setShare(bool on);
+    int setFuse(bool on);
+    int setPairStart(bool on);
+    int setProfile(bool on);
+    int shareStats(uint64_t* shared, uint64_t* restarted);
+    int fusedRows(uint64_t* rows);
+    // The slot engine runs every query from now on (autotuning).
+    void useSlots(bool on) { slotsOnly_ = on; }
+    // What the last run out of a packed database did (all zero otherwise).
+    const gv_resident_stats_t& residentStats() const { return res_; }
 
     // Mine every query; results in input order.  Queries with a plan error
     // get status GV_ERR_ARG; overflowing ones are re-run on the plain path.
@@ -79,11 +95,25 @@ public:
     // batch's own)
     std::map<std::string, uint32_t>& classTune() { return classIpt_; }
 
+    // Whether run() mines out of the packed form of the database, and the
+    // queries it then takes.
+    bool resident() const;
+    bool residentTakes(const CompiledQuery& cq) const {
+        return gv_resident_takes(g_, &cq.q, cq.hasLeaves ? &cq.leaves : nullptr) != 0;
+    }
+    gv_ctx_t context() const { return ctx_; }
+
 private:
+    int runResident(const std::vector<CompiledQuery>& qs, const std::vector<size_t>& order,
+                    std::vector<MineResult>& out, BatchStats& st);
+
     gv_ctx_t ctx_;
     gv_graph_t g_;
     PlainMiner* fallback_;
     BatchOptions opt_;
+    bool share_ = true, fuse_ = true, pairStart_ = true, profile_ = false, slotsOnly_ = false;
+    uint64_t resShared_ = 0, resFused_ = 0;
+    gv_resident_stats_t res_{};
     gv_batch_t b_ = nullptr;
     uint32_t nwords_ = 0;
     uint64_t rowCap_ = 0;

@@ -454,6 +454,12 @@ uint64_t gh_engine_graph_bytes(gh_engine_t e) {
     return b;
 }
 
+uint32_t gh_engine_resident_blocks(gh_engine_t e) {
+    uint32_t b = 0;
+    if (e && e->graph) gv_resident_info(e->graph, &b, nullptr);
+    return b;
+}
+
 int gh_engine_mine(gh_engine_t e, const char* text, int single_v, uint64_t* count,
                    uint64_t* alg_bytes, double* ms, uint32_t* bits, uint32_t nwords,
                    uint64_t* launches) {
@@ -662,52 +668,56 @@ int gh_engine_batch_profile(gh_engine_t e, int on) {
     if (!e) return GV_ERR_ARG;
     int rc = ensureBatch(e);
     if (rc != GV_OK) return rc;
-    return gv_batch_profile(e->batch->handle(), on);
+    return e->batch->setProfile(on != 0);
 }
 
 int gh_engine_batch_profile_bytes(gh_engine_t e, uint64_t* size_bytes, uint64_t* walk_bytes) {
     if (!e || !e->batch) return GV_ERR_ARG;
-    return gv_batch_profile_bytes(e->batch->handle(), size_bytes, walk_bytes);
+    gv_batch_t b;
+    int rc = e->batch->engine(&b);
+    return rc == GV_OK ? gv_batch_profile_bytes(b, size_bytes, walk_bytes) : rc;
 }
 
 int gh_engine_batch_pair_start(gh_engine_t e, int on) {
     if (!e) return GV_ERR_ARG;
     int rc = ensureBatch(e);
     if (rc != GV_OK) return rc;
-    return gv_batch_pair_start(e->batch->handle(), on);
+    return e->batch->setPairStart(on != 0);
 }
 
 int gh_engine_batch_share(gh_engine_t e, int on) {
     if (!e) return GV_ERR_ARG;
     int rc = ensureBatch(e);
     if (rc != GV_OK) return rc;
-    return gv_batch_share(e->batch->handle(), on);
+    return e->batch->setShare(on != 0);
 }
 
 int gh_engine_batch_share_stats(gh_engine_t e, uint64_t* shared, uint64_t* restarted) {
     if (!e) return GV_ERR_ARG;
     int rc = ensureBatch(e);
     if (rc != GV_OK) return rc;
-    return gv_batch_share_stats(e->batch->handle(), shared, restarted);
+    return e->batch->shareStats(shared, restarted);
 }
 
 int gh_engine_batch_fuse_sizing(gh_engine_t e, int on) {
     if (!e) return GV_ERR_ARG;
     int rc = ensureBatch(e);
     if (rc != GV_OK) return rc;
-    return gv_batch_fuse_sizing(e->batch->handle(), on);
+    return e->batch->setFuse(on != 0);
 }
 
 int gh_engine_batch_fused_rows(gh_engine_t e, uint64_t* rows) {
     if (!e) return GV_ERR_ARG;
     int rc = ensureBatch(e);
     if (rc != GV_OK) return rc;
-    return gv_batch_fused_rows(e->batch->handle(), rows);
+    return rows ? e->batch->fusedRows(rows) : GV_ERR_ARG;
 }
 
 int gh_engine_batch_history(gh_engine_t e, uint64_t* rows, uint64_t* candidates, uint32_t cap, uint32_t* n) {
     if (!e || !e->batch) return GV_ERR_ARG;
-    return gv_batch_history(e->batch->handle(), rows, candidates, cap, n);
+    gv_batch_t b;
+    int rc = e->batch->engine(&b);
+    return rc == GV_OK ? gv_batch_history(b, rows, candidates, cap, n) : rc;
 }
 
 int gh_engine_profile_records(gh_engine_t e, int* kinds, float* ms, uint64_t cap, uint64_t* n) {

@@ -456,7 +456,17 @@ int PlainMiner::mine(const CompiledQuery& cq, const Shard& sh, MineResult& out) 
             }
             counted = rc == GV_OK;
         } else if (rc == GV_OK && n) {
-            rc = runLevels(cq, rows, n, out);
+            // a whole query over a packed database: out of LDS, in one launch
+            rc = GV_ERR_CAPACITY;
+            if (sh.begin == 0 && sh.end == 0 && sh.stride == 1 && countByRows_) {
+                const gv_query_t* q = &cq.q;
+                const gv_leaves_t* lv = cq.hasLeaves ? &cq.leaves : nullptr;
+                uint32_t* bits = out.graphBits.data();
+                rc = gv_resident_mine(ctx_, g_, 1, &q, &lv, &out.count, &out.algBytes,
+                                      words ? &bits : nullptr, words, nullptr);
+                if (rc == GV_OK) out.launches++;
+            }
+            if (rc == GV_ERR_CAPACITY) rc = runLevels(cq, rows, n, out);
             counted = rc == GV_OK;
         }
         if (rc != GV_OK) {

@@ -104,6 +104,119 @@ private:
 };
 }  // namespace
 
+// Serving out of the packed form of a database: every loop turn takes the
+// requests that have arrived, as many as the engine has slots and the memory
+// bound admits, and mines them in one call, in which they share their common
+// steps.  A request the packed form does not take goes to the plain path.
+// A lone request waits kCompanyS for another: a launch costs both about
+// 30 us, and requests that arrive together are then one iteration, which the
+// memory bound splits.
+constexpr double kCompanyS = 20e-6;
+static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
+                         const std::vector<double>& arrivalS, uint64_t memBudget,
+                         const std::vector<uint64_t>& est, ServeResult& out, PlainMiner* side) {
+    const size_t n = reqs.size();
+    const uint32_t slots = bm.options().slots, nwords = out.nwords;
+    const Clock::time_point t0 = Clock::now();
+    SideWorker worker(side, reqs, t0);
+    std::vector<SideWorker::Done> sideDone;
+    std::vector<size_t> now;
+    std::vector<const gv_query_t*> q;
+    std::vector<const gv_leaves_t*> lv;
+    std::vector<uint64_t> count, bytes;
+    std::vector<uint32_t*> bits;
+    size_t next = 0, finished = 0;
+    auto finish = [&](size_t r, double atS) {
+        out.latencyMs[r] = (atS - arrivalS[r]) * 1e3;
+        ++finished;
+    };
+    // a request on the plain path
+    auto direct = [&](size_t r) {
+        ++out.direct;
+        if (worker.enabled()) {
+            worker.submit(r);
+            return (int)GV_OK;
+        }
+        MineResult mr;
+        if (!bm.fallback()) return (int)GV_ERR_CAPACITY;
+        const int rc = bm.fallback()->mine(reqs[r], mr);
+        if (rc != GV_OK) return rc;
+        out.counts[r] = mr.count;
+        std::copy(mr.graphBits.begin(), mr.graphBits.begin() + std::min<size_t>(mr.graphBits.size(), nwords),
+                  out.graphBits.begin() + r * (size_t)nwords);
+        finish(r, since(t0));
+        return (int)GV_OK;
+    };
+    while (finished < n) {
+        sideDone.clear();
+        worker.collect(sideDone);
+        for (auto& d : sideDone) {
+            if (d.status != GV_OK) return d.status;
+            out.counts[d.req] = d.count;
+            std::copy(d.bits.begin(), d.bits.begin() + std::min<size_t>(d.bits.size(), nwords),
+                      out.graphBits.begin() + d.req * (size_t)nwords);
+            finish(d.req, d.finishS);
+        }
+        now.clear();
+        uint64_t inUse = 0;
+        for (; next < n && now.size() < slots; ++next) {
+            if (arrivalS[next] > since(t0)) {
+                // nothing more has arrived; a lone, fresh request waits
+                if (now.size() != 1) break;
+                while (arrivalS[next] > since(t0) && since(t0) < arrivalS[now[0]] + kCompanyS) {
+                }
+                if (arrivalS[next] > since(t0)) break;
+            }
+            if (reqs[next].empty) {
+                finish(next, since(t0));
+            } else if (!bm.residentTakes(reqs[next])) {
+                const int rc = direct(next);
+                if (rc != GV_OK) return rc;
+            } else {
+                if (!now.empty() && inUse + est[next] > memBudget) break;
+                inUse += est[next];
+                now.push_back(next);
+            }
+        }
+        out.maxConcurrent = std::max<uint64_t>(out.maxConcurrent, now.size() + worker.pending());
+        out.maxBatched = std::max<uint64_t>(out.maxBatched, now.size());
+        if (now.empty()) {
+            if (finished >= n) break;
+            if (worker.pending() > 0) std::this_thread::sleep_for(std::chrono::microseconds(20));
+            else if (next < n) waitUntil(t0, arrivalS[next]);
+            continue;
+        }
+        const size_t m = now.size();
+        q.resize(m);
+        lv.resize(m);
+        count.resize(m);
+        bytes.resize(m);
+        bits.resize(m);
+        for (size_t i = 0; i < m; ++i) {
+            const CompiledQuery& cq = reqs[now[i]];
+            q[i] = &cq.q;
+            lv[i] = cq.hasLeaves ? &cq.leaves : nullptr;
+            bits[i] = out.graphBits.data() + now[i] * (size_t)nwords;
+        }
+        int rc = gv_resident_mine(bm.context(), bm.graph(), (uint32_t)m, q.data(), lv.data(), count.data(), bytes.data(),
+                                  nwords ? bits.data() : nullptr, nwords, nullptr);
+        if (rc == GV_ERR_CAPACITY) {
+            for (size_t r : now)
+                if ((rc = direct(r)) != GV_OK) return rc;
+            continue;
+        }
+        if (rc != GV_OK) return rc;
+        ++out.iterations;
+        const double t = since(t0);
+        for (size_t i = 0; i < m; ++i) {
+            out.counts[now[i]] = count[i];
+            finish(now[i], t);
+        }
+    }
+    out.wallS = since(t0) - (n ? arrivalS[0] : 0);
+    return GV_OK;
+}
+
 // A request whose estimated largest table exceeds a slot table's share
 // 1 / kDirectShare goes straight to the plain path.  The estimate (from label
 // statistics) runs low on the heaviest walk queries, which then overflow their
@@ -124,7 +237,6 @@ int serveBatched(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
     out = ServeResult();
     out.latencyMs.assign(n, 0);
     out.counts.assign(n, 0);
-    gv_batch_t b = bm.handle();
     const uint32_t slots = bm.options().slots;
     const uint64_t slotRowsBytes = bm.options().slotBytes;
     const uint32_t nwords = bm.graphWords();   // matched-graph bitset width
@@ -132,6 +244,10 @@ int serveBatched(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
     out.graphBits.assign(n * (size_t)nwords, 0);
     std::vector<uint64_t> est(n);
     for (size_t i = 0; i < n; ++i) est[i] = estimatePeakBytes(reqs[i], gs);
+    if (bm.resident()) return serveResident(bm, reqs, arrivalS, memBudget, est, out, side);
+    gv_batch_t b = nullptr;
+    rc = bm.engine(&b);
+    if (rc != GV_OK) return rc;
     std::vector<size_t> slotReq(slots, SIZE_MAX);
     std::vector<gv_slot_info_t> info(slots);
     size_t overflowed = 0;

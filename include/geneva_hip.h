@@ -278,6 +278,8 @@ typedef struct {
  * of 2^22 entries or more. */
 int gv_batch_create(gv_ctx_t ctx, gv_graph_t g, uint32_t slots, uint64_t slot_bytes,
                     uint64_t row_cap, const gv_tune_t* tune, gv_batch_t* out);
+/* GV_OK when gv_batch_create takes these settings (device memory aside). */
+int gv_batch_check(uint32_t slots, uint64_t slot_bytes, uint64_t row_cap, const gv_tune_t* tune);
 int gv_batch_destroy(gv_batch_t b);
 /* Rows sized per iteration from now on (at most the row_cap the batch was
  * created with; re-captures the iteration).  Slots whose table alone exceeds
@@ -376,6 +378,40 @@ int gv_batch_slot_iterations(gv_batch_t b, uint32_t slot, uint32_t* iterations);
 /* Slots, rows a slot table holds at a given width, free slots. */
 int gv_batch_info(gv_batch_t b, uint32_t* slots, uint64_t* slot_bytes, uint32_t* free_slots);
 
+/* ---- databases of small graphs, mined out of LDS ---------------------------
+ *
+ * gv_graph_set_owner also packs a database graph by graph into blocks that
+ * fit LDS, unless an edge joins two of its graphs, a graph packs to more than
+ * 64 KiB or the partitions times the labels exceed 256.  blocks: blocks of
+ * the packed form (0: the graph has none), bytes: its size in device memory. */
+int gv_resident_info(gv_graph_t g, uint32_t* blocks, uint64_t* bytes);
+
+/* 1 when gv_resident_mine mines this graph on this context: the graph is
+ * packed and byte-counting profiling (the table kernels') is off. */
+int gv_resident_ready(gv_ctx_t ctx, gv_graph_t g);
+
+typedef struct {
+    uint64_t launches;        /* mining launches */
+    uint64_t shared_queries;  /* queries that share their first steps with an earlier one */
+    uint64_t fused_rows;      /* rows read again for another step on the same table */
+    uint64_t rows;            /* rows read, shared ones once */
+    uint64_t bytes;           /* algorithmic bytes of the steps run, shared ones once */
+} gv_resident_stats_t;
+
+/* 1 when gv_resident_mine takes this query on this graph (whose leaf groups'
+ * products it keeps in 64 bits: leaves x log2 of the largest degree < 57). */
+int gv_resident_takes(gv_graph_t g, const gv_query_t* q, const gv_leaves_t* leaves);
+/* Mine n queries over every start vertex of a packed graph: counts,
+ * algorithmic bytes and, with bits (n pointers, each nullable), query i's
+ * matched graph ids in bits[i][0 .. nwords) (nwords = ceil(graphs / 32)).
+ * leaves (nullable, as its entries) as in gv_batch_admit_leaves.  Queries with
+ * the same first steps share them.  Synchronises.  GV_ERR_CAPACITY: not
+ * ready (gv_resident_ready), a query it does not take, or one whose tables and
+ * the largest block together exceed LDS. */
+int gv_resident_mine(gv_ctx_t ctx, gv_graph_t g, uint32_t n, const gv_query_t* const* queries,
+                     const gv_leaves_t* const* leaves, uint64_t* counts, uint64_t* alg_bytes,
+                     uint32_t* const* bits, uint32_t nwords, gv_resident_stats_t* stats);
+
 /* Per-kernel profiling on the context's stream.  on = 1: every launch is
  * bracketed by HIP events; on = 2: in addition each kernel kind counts the
  * bytes its algorithm reads and writes (each access once) and its work units
@@ -396,6 +432,7 @@ int gv_batch_info(gv_batch_t b, uint32_t* slots, uint64_t* slot_bytes, uint32_t*
 #define GV_KIND_ROWS 5
 #define GV_KIND_ISECT 6
 #define GV_KIND_CHAIN 7
+#define GV_KIND_RESIDENT 9   /* gv_resident_mine: its mining launch */
 int gv_profile_enable(gv_ctx_t ctx, int on);
 int gv_profile_reset(gv_ctx_t ctx);
 int gv_profile_read(gv_ctx_t ctx, int kind, uint64_t* launches, double* total_ms,
@@ -404,7 +441,8 @@ int gv_profile_read(gv_ctx_t ctx, int kind, uint64_t* launches, double* total_ms
  * candidates (extend, count); 0 for batch iterations (extents on the device). */
 int gv_profile_units(gv_ctx_t ctx, int kind, uint64_t* units);
 /* Algorithmic bytes B (the reference figure, accumulated exactly as for the
- * counters) of a kind since the last reset, with on = 2. */
+ * counters) of a kind since the last reset, with on = 2 (GV_KIND_RESIDENT:
+ * of its steps, shared ones once, with on = 1). */
 int gv_profile_alg_bytes(gv_ctx_t ctx, int kind, uint64_t* bytes);
 
 /* Every profiled launch since the last reset, in launch order: its kind and

@@ -86,6 +86,8 @@ gh_engine_t gh_engine_create(gh_dataset_t ds, int device, uint64_t level_bytes, 
 void gh_engine_free(gh_engine_t e);
 /* Device bytes of the resident graph. */
 uint64_t gh_engine_graph_bytes(gh_engine_t e);
+/* Blocks of a database's packed form (gv_resident_info); 0: it has none. */
+uint32_t gh_engine_resident_blocks(gh_engine_t e);
 /* Mine one query on the plain path (one query per launch sequence).
  * graph_bits (nullable) receives ceil(ngraphs/32) words. */
 int gh_engine_mine(gh_engine_t e, const char* query_text, int single_v, uint64_t* count,
