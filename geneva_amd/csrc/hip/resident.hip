@@ -20,9 +20,10 @@
 // the waves a CU holds (its LDS) and how evenly they are kept busy.  Measured
 // on MI355X, calls on three seeds each, before = the table engines (a launch
 // or more per step of a query, tables in HBM):
-//   one query on 400 / 20,000 graphs of 100 edges    860 -> 380 us for 24, 4.7 -> 2.0 ms for 24
-//   131 queries on 20,000 graphs                     3.3 -> 2.0 ms
-//   256 queries on 100,000 graphs                    17.9 -> 9.2 ms
+//   10 queries on 1,000 small graphs, one by one      939 ->  380 us
+//   24 queries on 20,000 graphs, one by one          4532 -> 1957 us
+//   131 queries on 17,321 graphs, one call           3.08 -> 1.77 ms
+//   256 queries on 100,000 graphs, one call          16.9 -> 9.24 ms
 // The split of the work that gives these: workgroups take blocks as they
 // become free (with every gridDim-th block 3.05 and 11.1 ms), their waves take
 // tasks of a block, and a wave without a task gets half of the next table that
