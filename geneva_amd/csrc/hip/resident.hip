@@ -28,7 +28,7 @@
 // become free (with every gridDim-th block 3.05 and 11.1 ms), their waves take
 // tasks of a block, and a wave without a task gets half of the next table that
 // another one makes: one start vertex can hold most of a block's work (without
-// this 3.1 and 10.0 ms; one block of seed 102 kept a single wave at work for
+// this 3.1 and 10.0 ms; one block of one database kept a single wave at work for
 // 3.4 of 4.0 ms).
 #include "common.h"
 
@@ -301,7 +301,10 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
     };
     for (uint32_t bi = blockIdx.x; bi < a.nblk;) {
         const RBlk blk = a.blk[bi];
-        uint32_t then = bi;   // the workgroup's next block
+        // The workgroup's next block: the next free one, or for one small
+        // query, whose blocks take a few us each, at a fixed stride (the
+        // counter's atomics come back about 100 ns apart, from all XCDs in turn).
+        uint32_t then = bi;
         if (!kSmall && threadIdx.x == 0) then = atomicAdd(a.next, 1u);
         for (uint32_t i = threadIdx.x; i < blk.n16; i += blockDim.x) rlds[i] = a.img[(uint64_t)blk.off16 + i];
         if (threadIdx.x == 0) {
@@ -1334,7 +1337,7 @@ int gv_resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* con
         if (!small) {
             // the split of a CU's LDS that holds the most waves, in two
             // workgroups or more: one alone idles at each change of block
-            // (131 queries, seed 100: two of 4 waves 1.72 ms, one of 8 2.14;
+            // (131 queries, one database: two of 4 waves 1.72 ms, one of 8 2.14;
             // 256 queries: two of 8 8.75, two of 4 13.9)
             waves = 0;
             uint32_t most = 0;
