@@ -1211,11 +1211,18 @@ bool valid_query(const gv_query_t& q, const gv_graph* g) {
 int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
     if (!c->resw) c->resw = new ResWork();
     ResWork* w = c->resw;
+    // (each of the two on its own: a call that found memory for one of them
+    // only leaves that one for the next)
     if (!w->d_acc) {
-        if (hipMalloc(&w->d_acc, 16 * kRMaxOps * kRLines + 16) != hipSuccess ||
-            hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps, hipHostMallocCoherent) != hipSuccess)
+        if (hipMalloc(&w->d_acc, 16 * kRMaxOps * kRLines + 16) != hipSuccess) {
+            w->d_acc = nullptr;
             return GV_ERR_NOMEM;
+        }
         w->dirty = true;
+    }
+    if (!w->h_acc && hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps, hipHostMallocCoherent) != hipSuccess) {
+        w->h_acc = nullptr;
+        return GV_ERR_NOMEM;
     }
     if (prog > w->prog_cap) {
         HIPCHK(hipStreamSynchronize(c->stream));

@@ -1,0 +1,88 @@
+// Host side of the packed databases (gv_graph_set_owner, gv_resident_mine)
+// without a device: one case a run, named by the first argument.
+#include "fake_hip.h"
+#include "geneva_hip.h"
+
+namespace {
+
+int fails = 0;
+#define CHECK(x)                                                    \
+    do {                                                            \
+        if (!(x)) {                                                 \
+            std::printf("line %d: not so: %s\n", __LINE__, #x);     \
+            ++fails;                                                \
+        }                                                           \
+    } while (0)
+
+// two graphs of one edge each: vertices 1-2 and 3-4, labels 1 and 2
+const uint32_t kLabels[] = {4, 1, 2, 1, 2};
+const uint32_t kBlock[] = {18, 4, 1, 0, 9, /*sources*/ 1, 0, 4, 0, /*lists*/ 0, 1, 2, 3, 4, /*neighbours*/ 2, 1, 4, 3};
+const uint32_t kOwner[] = {0, 0, 0, 1, 1};
+
+struct Db {
+    gv_ctx_t c = nullptr;
+    gv_graph_t g = nullptr;
+    explicit Db(int device = 0) {
+        const uint32_t* blocks[] = {kBlock};
+        const uint32_t edge_label = 1;
+        CHECK(gv_ctx_create(device, &c) == GV_OK);
+        CHECK(gv_graph_create(c, kLabels, 1, blocks, &edge_label, &g) == GV_OK);
+    }
+    ~Db() {
+        gv_graph_destroy(g);
+        gv_ctx_destroy(c);
+    }
+    int mine() {
+        gv_query_t q{};
+        q.k = 2;
+        q.step[1].label = 1;
+        q.step[1].col = 1;
+        q.step[1].nback = 1;
+        q.step[1].restrict_col = GV_NONE;
+        const gv_query_t* qs[] = {&q};
+        uint64_t count = 0, bytes = 0;
+        uint32_t word = 0, *bits[] = {&word};
+        return gv_resident_mine(c, g, 1, qs, nullptr, &count, &bytes, bits, 1, nullptr);
+    }
+};
+
+// accumulators that a call adds to start at zero, and results have a place
+hipError_t accumulators(const std::string& name, void** args) {
+    if (name.find("k_resident_out") == std::string::npos) return hipSuccess;
+    const char* acc = *(char**)args[0];
+    const uint32_t nacc = *(uint32_t*)args[1];
+    CHECK(*(void**)args[2] != nullptr);
+    bool zero = acc != nullptr;
+    for (uint32_t i = 0; zero && i < 8 * nacc; ++i) zero = acc[i] == 0;
+    CHECK(zero);
+    return hipSuccess;
+}
+
+// After a call that found no memory the next one works.
+void failed_allocation() {
+    fake::on_launch = accumulators;
+    for (int i = 0;; ++i) {
+        Db db;
+        CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+        fake::failed = false;
+        fake::fail_alloc = i;
+        const int first = db.mine();
+        fake::fail_alloc = -1;
+        std::printf("allocation %d: %d\n", i, first);
+        std::fflush(stdout);
+        CHECK(fake::failed == (first != GV_OK));
+        CHECK(db.mine() == GV_OK);
+        if (!fake::failed) break;
+        CHECK(i < 100);
+    }
+}
+
+}  // namespace
+
+int main(int, char** argv) {
+    const std::string what = argv[1];
+    if (what == "failed_allocation") failed_allocation();
+    else return 2;
+    std::printf("%s: %d wrong\n", what.c_str(), fails);
+    return fails ? 1 : 0;
+}
