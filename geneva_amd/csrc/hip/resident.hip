@@ -1306,7 +1306,12 @@ int gv_resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* con
         if (!small) make_tasks(p, R);
         const uint64_t tb = sizeof(RTask) * p.tasks.size();
         const uint64_t nb = bits ? (uint64_t)p.nterms * nwords : 0;
-        int rc = res_buffers(c, small ? 0 : pb + tb, nb);
+        const int rc = res_buffers(c, small ? 0 : pb + tb, nb);
+        if (rc == GV_ERR_NOMEM) {
+            // the table engines may have what they need already
+            (void)hipGetLastError();
+            return GV_ERR_CAPACITY;
+        }
         if (rc != GV_OK) return rc;
         ResWork* w = c->resw;
         RArgs a;

@@ -406,8 +406,9 @@ int gv_resident_takes(gv_graph_t g, const gv_query_t* q, const gv_leaves_t* leav
  * matched graph ids in bits[i][0 .. nwords) (nwords = ceil(graphs / 32)).
  * leaves (nullable, as its entries) as in gv_batch_admit_leaves.  Queries with
  * the same first steps share them.  Synchronises.  GV_ERR_CAPACITY: not
- * ready (gv_resident_ready), a query it does not take, or one whose tables and
- * the largest block together exceed LDS. */
+ * ready (gv_resident_ready), a query it does not take, one whose tables and
+ * the largest block together exceed LDS, or no memory for its buffers: the
+ * table engines mine the queries then. */
 int gv_resident_mine(gv_ctx_t ctx, gv_graph_t g, uint32_t n, const gv_query_t* const* queries,
                      const gv_leaves_t* const* leaves, uint64_t* counts, uint64_t* alg_bytes,
                      uint32_t* const* bits, uint32_t nwords, gv_resident_stats_t* stats);

@@ -77,11 +77,31 @@ void failed_allocation() {
     }
 }
 
+// A call that finds no memory says what a database that does not fit says
+// (the caller's table engines mine it), and leaves no error behind.
+void no_memory_is_capacity() {
+    fake::sticky = true;
+    for (int i = 0;; ++i) {
+        Db db;
+        CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+        fake::failed = false;
+        fake::fail_alloc = i;
+        const int first = db.mine();
+        fake::fail_alloc = -1;
+        CHECK(first == (fake::failed ? GV_ERR_CAPACITY : GV_OK));
+        CHECK(fake::last == hipSuccess);
+        CHECK(db.mine() == GV_OK);
+        if (!fake::failed) break;
+        CHECK(i < 100);
+    }
+}
+
 }  // namespace
 
 int main(int, char** argv) {
     const std::string what = argv[1];
     if (what == "failed_allocation") failed_allocation();
+    else if (what == "no_memory_is_capacity") no_memory_is_capacity();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
