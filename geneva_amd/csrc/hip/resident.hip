@@ -744,6 +744,7 @@ void res_image_free(gv_graph* g) {
     if (!r) return;
     if (r->d_blk) (void)hipFree(r->d_blk);
     if (r->d_img) (void)hipFree(r->d_img);
+    g->dev_bytes -= r->bytes;
     delete r;
     g->res = nullptr;
 }
@@ -863,6 +864,7 @@ int res_image_build(gv_graph* g, const uint32_t* graph_of) {
     }
     g->res = r.release();
     ResImage* R = g->res;
+    g->dev_bytes += R->bytes;
     HIPCHK(hipMemcpy(R->d_blk, blks.data(), sizeof(RBlk) * blks.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(dord.p, ord.data(), 4 * nlab, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(dpos.p, pos.data(), 4 * nv1, hipMemcpyHostToDevice));
@@ -873,7 +875,6 @@ int res_image_build(gv_graph* g, const uint32_t* graph_of) {
     const int most = kRLdsMost;
     HIPCHK(hipFuncSetAttribute((const void*)k_resident<true>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     HIPCHK(hipFuncSetAttribute((const void*)k_resident<false>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
-    g->dev_bytes += R->bytes;
     return GV_OK;
 }
 

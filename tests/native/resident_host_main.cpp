@@ -96,12 +96,59 @@ void no_memory_is_capacity() {
     }
 }
 
+// What packing needs of its kernels: labels, and one segment with one
+// neighbour for each vertex.
+hipError_t pack_kernels(const std::string& name, void** args) {
+    if (name.find("k_pack_labels") != std::string::npos) {
+        const uint32_t* lverts = *(uint32_t**)args[0];
+        const uint64_t n = *(uint64_t*)args[1], *lvoff = *(uint64_t**)args[2];
+        const uint32_t nl = *(uint32_t*)args[3];
+        uint32_t* lab = *(uint32_t**)args[4];
+        for (uint32_t l = 0; l < nl; ++l)
+            for (uint64_t i = lvoff[l]; i < lvoff[l + 1] && i < n; ++i) lab[lverts[i]] = l;
+    } else if (name.find("k_pack_count") != std::string::npos) {
+        const uint64_t nv1 = *(uint64_t*)args[2];
+        for (int a : {3, 4})
+            for (uint64_t v = 1; v < nv1; ++v) (*(uint32_t**)args[a])[v] = 1;
+    }
+    return hipSuccess;
+}
+uint64_t device_bytes(gv_graph_t g) {
+    uint64_t b = 0;
+    CHECK(gv_graph_info(g, nullptr, nullptr, nullptr, nullptr, &b) == GV_OK);
+    return b;
+}
+uint64_t packed_bytes(gv_graph_t g) {
+    uint32_t blocks = 0;
+    uint64_t b = 0;
+    CHECK(gv_resident_info(g, &blocks, &b) == GV_OK);
+    CHECK((blocks == 0) == (b == 0));
+    return b;
+}
+
+// The packed form counts once in a graph's bytes, however often its owners are set.
+void owners_twice() {
+    fake::on_launch = pack_kernels;
+    Db db;
+    const uint64_t bare = device_bytes(db.g);
+    for (int i = 0; i < 3; ++i) {
+        CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+        CHECK(packed_bytes(db.g) > 0);
+        CHECK(device_bytes(db.g) == bare + packed_bytes(db.g));
+    }
+    const uint32_t one[5] = {};   // one graph is not packed
+    CHECK(gv_graph_set_owner(db.g, one, 1) == GV_OK);
+    CHECK(packed_bytes(db.g) == 0);
+    CHECK(device_bytes(db.g) == bare);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
     const std::string what = argv[1];
     if (what == "failed_allocation") failed_allocation();
     else if (what == "no_memory_is_capacity") no_memory_is_capacity();
+    else if (what == "owners_twice") owners_twice();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
