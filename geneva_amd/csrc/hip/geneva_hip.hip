@@ -1361,6 +1361,7 @@ int gv_graph_set_owner(gv_graph_t g, const uint32_t* graph_of, uint32_t ngraphs)
     if (!g || !graph_of || ngraphs == 0) return GV_ERR_ARG;
     for (uint64_t v = 0; v < g->nv1; ++v)
         if (graph_of[v] >= ngraphs) return GV_ERR_ARG;
+    HIPCHK(hipSetDevice(g->ctx->device));
     if (g->d_gof) HIPCHK(hipFree(g->d_gof));
     g->d_gof = nullptr;
     if (hipMalloc(&g->d_gof, g->nv1 * sizeof(uint32_t)) != hipSuccess) return GV_ERR_NOMEM;

@@ -142,6 +142,19 @@ void owners_twice() {
     CHECK(device_bytes(db.g) == bare);
 }
 
+// Packing runs on the graph's device, whichever the calling thread used last.
+hipError_t on_device_1(const std::string& name, void** args) {
+    CHECK(fake::device == 1);
+    return pack_kernels(name, args);
+}
+void owners_on_their_device() {
+    Db db(1);
+    fake::on_launch = on_device_1;
+    fake::device = 0;
+    CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+    CHECK(packed_bytes(db.g) > 0);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -149,6 +162,7 @@ int main(int, char** argv) {
     if (what == "failed_allocation") failed_allocation();
     else if (what == "no_memory_is_capacity") no_memory_is_capacity();
     else if (what == "owners_twice") owners_twice();
+    else if (what == "owners_on_their_device") owners_on_their_device();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;

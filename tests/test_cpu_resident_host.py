@@ -27,7 +27,8 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["failed_allocation", "no_memory_is_capacity", "owners_twice"])
+@pytest.mark.parametrize("case", ["failed_allocation", "no_memory_is_capacity", "owners_twice",
+                                  "owners_on_their_device"])
 def test_resident_host(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
