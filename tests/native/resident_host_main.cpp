@@ -155,6 +155,37 @@ void owners_on_their_device() {
     CHECK(packed_bytes(db.g) > 0);
 }
 
+// Owners are set also where the database cannot be packed: a launch of the
+// packing fails, or a device allocation of its own.
+int fail_launch = -1;
+hipError_t some_launch_fails(const std::string& name, void** args) {
+    if (fail_launch >= 0 && fail_launch-- == 0) {
+        fake::failed = true;
+        return hipErrorLaunchFailure;
+    }
+    return pack_kernels(name, args);
+}
+void packing_fails() {
+    fake::on_launch = some_launch_fails;
+    fake::sticky = true;
+    for (int what = 0; what < 2; ++what)
+        for (int i = 0;; ++i) {
+            Db db;
+            fake::failed = false;
+            // allocation 0 is the owners' own
+            (what ? fail_launch : fake::fail_alloc) = i + (what ? 0 : 1);
+            CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+            fail_launch = fake::fail_alloc = -1;
+            CHECK(fake::last == hipSuccess);
+            uint32_t n = 0;
+            CHECK(gv_graph_owners(db.g, &n) == GV_OK && n == 2);
+            CHECK((packed_bytes(db.g) == 0) == fake::failed);
+            CHECK(db.mine() == (fake::failed ? GV_ERR_CAPACITY : GV_OK));
+            if (!fake::failed) break;
+            CHECK(i < 100);
+        }
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -163,6 +194,7 @@ int main(int, char** argv) {
     else if (what == "no_memory_is_capacity") no_memory_is_capacity();
     else if (what == "owners_twice") owners_twice();
     else if (what == "owners_on_their_device") owners_on_their_device();
+    else if (what == "packing_fails") packing_fails();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
