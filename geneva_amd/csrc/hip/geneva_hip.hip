@@ -1367,7 +1367,13 @@ int gv_graph_set_owner(gv_graph_t g, const uint32_t* graph_of, uint32_t ngraphs)
     if (hipMalloc(&g->d_gof, g->nv1 * sizeof(uint32_t)) != hipSuccess) return GV_ERR_NOMEM;
     HIPCHK(hipMemcpy(g->d_gof, graph_of, g->nv1 * sizeof(uint32_t), hipMemcpyHostToDevice));
     g->ngraphs = ngraphs;
-    if (res_image_build(g, graph_of) != GV_OK) {
+    int rc;
+    try {
+        rc = res_image_build(g, graph_of);
+    } catch (const std::bad_alloc&) {
+        rc = GV_ERR_NOMEM;
+    }
+    if (rc != GV_OK) {
         // the owners are set; without the packed form the table engines mine
         // the database
         res_image_free(g);

@@ -1256,27 +1256,9 @@ int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
     return GV_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int gv_resident_info(gv_graph_t g, uint32_t* blocks, uint64_t* bytes) {
-    if (!g) return GV_ERR_ARG;
-    if (blocks) *blocks = g->res ? g->res->nblk : 0;
-    if (bytes) *bytes = g->res ? g->res->bytes : 0;
-    return GV_OK;
-}
-
-int gv_resident_ready(gv_ctx_t c, gv_graph_t g) { return c && g && g->res && !c->prof_bytes ? 1 : 0; }
-
-int gv_resident_takes(gv_graph_t g, const gv_query_t* q, const gv_leaves_t* leaves) {
-    if (!g || !q || !valid_query(*q, g) || (leaves && (!valid_leaves(leaves, g) || leaves->k != q->k))) return 0;
-    return g->res && (!leaves || leaves_fit(*leaves, g)) ? 1 : 0;
-}
-
-int gv_resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const* qs,
-                     const gv_leaves_t* const* leaves, uint64_t* counts, uint64_t* alg_bytes,
-                     uint32_t* const* bits, uint32_t nwords, gv_resident_stats_t* stats) {
+int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const* qs,
+                  const gv_leaves_t* const* leaves, uint64_t* counts, uint64_t* alg_bytes,
+                  uint32_t* const* bits, uint32_t nwords, gv_resident_stats_t* stats) {
     if (!c || !g || (n && (!qs || !counts || !alg_bytes))) return GV_ERR_ARG;
     if (bits && nwords != (g->ngraphs + 31) / 32) return GV_ERR_ARG;
     for (uint32_t i = 0; i < n; ++i) {
@@ -1408,6 +1390,37 @@ int gv_resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* con
     if (c->prof) c->res_bytes += st.bytes;
     if (stats) *stats = st;
     return GV_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int gv_resident_info(gv_graph_t g, uint32_t* blocks, uint64_t* bytes) {
+    if (!g) return GV_ERR_ARG;
+    if (blocks) *blocks = g->res ? g->res->nblk : 0;
+    if (bytes) *bytes = g->res ? g->res->bytes : 0;
+    return GV_OK;
+}
+
+int gv_resident_ready(gv_ctx_t c, gv_graph_t g) { return c && g && g->res && !c->prof_bytes ? 1 : 0; }
+
+int gv_resident_takes(gv_graph_t g, const gv_query_t* q, const gv_leaves_t* leaves) {
+    if (!g || !q || !valid_query(*q, g) || (leaves && (!valid_leaves(leaves, g) || leaves->k != q->k))) return 0;
+    return g->res && (!leaves || leaves_fit(*leaves, g)) ? 1 : 0;
+}
+
+int gv_resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const* qs,
+                     const gv_leaves_t* const* leaves, uint64_t* counts, uint64_t* alg_bytes,
+                     uint32_t* const* bits, uint32_t nwords, gv_resident_stats_t* stats) {
+    try {
+        return resident_mine(c, g, n, qs, leaves, counts, alg_bytes, bits, nwords, stats);
+    } catch (const std::bad_alloc&) {
+        // no host memory, as without device memory: the table engines may do.
+        // A launch may still be running with this call's buffers.
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return GV_ERR_HIP;
+        return GV_ERR_CAPACITY;
+    }
 }
 
 }  // extern "C"

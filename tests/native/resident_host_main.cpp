@@ -3,6 +3,22 @@
 #include "fake_hip.h"
 #include "geneva_hip.h"
 
+#include <new>
+
+// host allocations until one throws (-1: none does)
+static int fail_new = -1;
+static bool new_failed = false;
+void* operator new(size_t n) {
+    if (fail_new >= 0 && fail_new-- == 0) {
+        new_failed = true;
+        throw std::bad_alloc();
+    }
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 namespace {
 
 int fails = 0;
@@ -186,6 +202,27 @@ void packing_fails() {
         }
 }
 
+// No exception leaves the library: without host memory to pack in a database
+// stays unpacked, without host memory for a call the table engines mine it.
+void no_host_memory() {
+    fake::on_launch = pack_kernels;
+    for (int what = 0; what < 2; ++what)
+        for (int i = 0;; ++i) {
+            Db db;
+            if (what) CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+            new_failed = false;
+            fail_new = i;
+            const int rc = what ? db.mine() : gv_graph_set_owner(db.g, kOwner, 2);
+            fail_new = -1;
+            CHECK(rc == (what && new_failed ? GV_ERR_CAPACITY : GV_OK));
+            uint32_t n = 0;
+            CHECK(gv_graph_owners(db.g, &n) == GV_OK && n == 2);
+            CHECK(db.mine() == (packed_bytes(db.g) ? GV_OK : GV_ERR_CAPACITY));
+            if (!new_failed) break;
+            CHECK(i < 1000);
+        }
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -195,6 +232,7 @@ int main(int, char** argv) {
     else if (what == "owners_twice") owners_twice();
     else if (what == "owners_on_their_device") owners_on_their_device();
     else if (what == "packing_fails") packing_fails();
+    else if (what == "no_host_memory") no_host_memory();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
