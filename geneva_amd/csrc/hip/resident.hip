@@ -29,7 +29,8 @@
 // tasks of a block, and a wave without a task gets half of the next table that
 // another one makes: one start vertex can hold most of a block's work (without
 // this 3.1 and 10.0 ms; one block of one database kept a single wave at work for
-// 3.4 of 4.0 ms).
+// 3.4 of 4.0 ms).  What a block holds beyond its share goes to the whole chip
+// in another launch (kRSpare).
 #include "common.h"
 
 #include <memory>
@@ -108,7 +109,7 @@ struct RBlk {
 struct RArgs {
     const RBlk* blk;
     const uint4* img;
-    uint32_t nblk, mask_words;
+    uint32_t mask_words;
     // the program (RProg::image; its list of leaf steps' columns begins at
     // o_col bytes); tasks (kSmall: task t is operation 0 on rows [64 t,
     // 64 (t + 1)) of label0)
@@ -124,7 +125,15 @@ struct RArgs {
     // embeddings); kRLines copies of 2 nops words, block b adds to copy b mod
     // kRLines
     unsigned long long* acc;
-    uint32_t* next;              // blocks handed out beyond the first of each workgroup (not kSmall)
+    uint32_t* next;              // blocks handed out beyond the first of each workgroup
+    // tables set aside (kAside...), to read and to write: item_words each
+    uint32_t nwork;              // blocks, or with `items` tables to take up
+    uint32_t item_words;
+    const uint32_t* items;       // set aside by the launch before
+    uint32_t* aside;             // for the next launch: `naside` of at most aside_cap
+    uint32_t* naside;
+    uint32_t aside_cap;
+    uint32_t budget;             // batches a wave works through in a block before it sets tables aside (below 2^31)
     uint32_t* bits;              // nterms x nwords (nullable)
     uint32_t prog[kRSmallBytes / 4];   // a small program
 };
@@ -138,11 +147,39 @@ constexpr uint32_t kRLeastRows = 16;             // start rows of a share
 constexpr uint32_t kRLdsMost = 160u << 10;       // LDS of a CU
 constexpr uint32_t kRSmallWaves = 4, kRWaves = 8;   // waves of a workgroup, at most
 constexpr uint32_t kRGive = 16;                  // rows of a table worth sharing; 4 or 48: within 2%
+constexpr uint64_t kRAsideBytes = 4u << 20;      // tables set aside by one launch, at most
+// A wave's work in a block, in batches of 64 rows and of 64 candidates, before
+// it sets tables aside: kRSpare (about 80 us of a wave alone) and the mean over
+// the waves that the label statistics let expect.  The blocks of a batch are
+// handed out one by one, so there it first looks again every kRAgain whether
+// any is left, and works through kRTail after the last.  What is set aside
+// costs another launch and a synchronisation (35 us) and its block's image
+// again.  Calls on databases with hubs, without and with it, and with the
+// table engines:
+//   a star query on 6,000 graphs of 20-400 vertices       1330 ->  342 us  ( 285)
+//   200 queries on the same, one call                     3.21 -> 1.76 ms  (3.48)
+//   9 queries on 8 graphs of 1,450 vertices, one by one   1746 ->  933 us  (1448)
+//   9 on 20,000 small and 10 such graphs, one by one      2589 -> 1024 us  (2637)
+// 600 queries, one by one, on two databases without such hubs: the sum within
+// 1%, on one with them 6% less; batches of 24 to 600 of them 3% more to 43%
+// less.  With kRSpare 100 / 200 / 300 the heaviest of the 600 took 472 / 548 /
+// 602 us; without kRTail batches that end evenly were up to 10% slower.
+constexpr double kRSpare = 160;
+constexpr uint32_t kRTail = 256, kRAgain = 64;
 // a workgroup's control words: tasks taken, next block, waves waiting for a
 // share (a bit each), waves at work; then each wave's share: given | first
 // operation | rows, width << 16 | operations left on a width-2 table
 enum { kCtlTask = 0, kCtlNext = 4, kCtlIdle = 8, kCtlBusy = 12, kCtlShare = 16 };
 constexpr uint32_t kRCtlBytes = kCtlShare + 16 * kRWaves;
+
+// A table set aside: a wave that has done much in one block leaves the next
+// tables it makes to the whole chip, in another launch (a rare star's centre
+// can hold nearly all of a query's work, in one block of a thousand).  Words:
+// block, first operation, rows | width << 16, operations left on a width-2
+// table, first column (bytes), columns; from kRAside on the columns, kRCap
+// 16-bit numbers each.
+enum { kAsideBlock = 0, kAsideOp = 1, kAsideRows = 2, kAsideLeft = 3, kAsideCol = 4, kAsideCols = 5, kRAside = 8 };
+static_assert(kRCap == 128, "a wave moves a column with one word a lane");
 
 extern __shared__ uint4 rlds[];
 
@@ -166,6 +203,18 @@ __device__ __forceinline__ void st32_shared(uint32_t o, uint32_t v) {
 }
 
 __device__ __forceinline__ uint32_t uni(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+// x in a vector register: k_resident's scalar registers are all taken, so what
+// is seldom read does not live in one (uni gets it back)
+__device__ __forceinline__ uint32_t vec(uint32_t x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+// the kernel's arguments, read where they are used and not before
+__device__ __forceinline__ const GV_CONST RArgs& rargs() {
+    const GV_CONST char* p = (const GV_CONST char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const GV_CONST RArgs*)p;
+}
 
 // LDS written by other lanes of this wave is visible after it
 __device__ __forceinline__ void wave_lds_sync() {
@@ -278,13 +327,13 @@ __device__ __forceinline__ uint64_t rleaf_count(const RView& V, const GV_CONST R
 // One workgroup takes blocks of the database; its waves take the block's
 // tasks (a width-1 operation and a range of its start vertices) and run each
 // down the trie.
-template <bool kSmall>
+// kAside: what it takes are the tables set aside by the launch before.
+template <bool kSmall, bool kAside>
 __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
     const GV_CONST char* ops;
     if constexpr (kSmall) ops = (const GV_CONST char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RArgs, prog);
     else ops = (const GV_CONST char*)a.ops;
     const GV_CONST RTask* tasks = (const GV_CONST RTask*)a.tasks;
-    const GV_CONST uint32_t* leaf_cols = (const GV_CONST uint32_t*)(ops + a.o_col);
     const uint32_t lane = __lane_id(), wib = uni(threadIdx.x >> 6);
     const uint32_t o_acc = a.img_bytes, o_bits = o_acc + 16 * a.nops;
     const uint32_t o_ctl = (o_bits + 4 * a.nterms * a.gw + 15) & ~15u;
@@ -299,14 +348,20 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
         atomicOr(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(rlds) + o_bits + 4 * (term * a.gw + (g >> 5))),
                  1u << (g & 31));
     };
-    for (uint32_t bi = blockIdx.x; bi < a.nblk;) {
+    uint32_t loaded = kNone;
+    for (uint32_t wi = blockIdx.x; wi < a.nwork;) {
+        const uint32_t wv = vec(wi);
+        const uint32_t bi = kAside ? uni(a.items[(uint64_t)wi * a.item_words]) : wi;
         const RBlk blk = a.blk[bi];
         // The workgroup's next block: the next free one, or for one small
         // query, whose blocks take a few us each, at a fixed stride (the
         // counter's atomics come back about 100 ns apart, from all XCDs in turn).
-        uint32_t then = bi;
-        if (!kSmall && threadIdx.x == 0) then = atomicAdd(a.next, 1u);
-        for (uint32_t i = threadIdx.x; i < blk.n16; i += blockDim.x) rlds[i] = a.img[(uint64_t)blk.off16 + i];
+        uint32_t then = 0;
+        constexpr bool counter = !kSmall || kAside;   // tables set aside differ too much for a stride
+        if (counter && threadIdx.x == 0) then = atomicAdd(a.next, 1u);
+        if (!kAside || bi != loaded)
+            for (uint32_t i = threadIdx.x; i < blk.n16; i += blockDim.x) rlds[i] = a.img[(uint64_t)blk.off16 + i];
+        if constexpr (kAside) loaded = bi;
         if (threadIdx.x == 0) {
             st32(o_ctl + kCtlTask, 0);
             st32(o_ctl + kCtlIdle, 0);
@@ -318,6 +373,8 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
         V.nbr = V.doff + 2 * (blk.ndir + 1);
         const uint32_t o_lv = V.nbr + 2 * blk.ne, o_lvo = o_lv + 2 * blk.nv;
         __syncthreads();
+        uint32_t spare = vec(a.budget);   // batches before this wave sets tables aside (as int)
+        uint32_t tail = vec(0);           // whether no block was left when it last looked
         bool drained = false;   // no task is left: this wave takes shares of the others' work
         for (;;) {
             uint32_t opo, n;              // the operation, and rows of the table it reads
@@ -329,21 +386,38 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                 uint32_t t = 0;
                 if (lane == 0) t = atomicAdd(lds_word(o_ctl + kCtlTask), 1u);
                 t = uni(t);
-                if (t >= a.ntasks) {
+                if (t >= (kAside ? blockDim.x >> 6 : a.ntasks)) {
                     drained = true;
                     continue;
                 }
-                RTask task;
-                if constexpr (kSmall) task = RTask{0, a.label0, 64 * t, 64, kNone, 0, 1, 0};
-                else task = {tasks[t].op, tasks[t].label, tasks[t].first, tasks[t].rows, tasks[t].child, tasks[t].nchild, tasks[t].account, 0};
-                opo = task.op;
-                child = task.child;
-                nchild = task.nchild;
-                account = task.account;
-                const uint32_t s0 = uni(ld16(o_lvo + 2 * task.label)) + task.first, s1 = uni(ld16(o_lvo + 2 * task.label + 2));
-                if (s0 >= s1) continue;
-                n = s1 - s0 < task.rows ? s1 - s0 : task.rows;
-                for (uint32_t i = lane; i < n; i += 64) st16(V.wv + 2 * i, ld16(o_lv + 2 * (s0 + i)));
+                if constexpr (kAside) {
+                    const uint32_t* item = a.items + (uint64_t)uni(wv) * a.item_words;
+                    opo = uni(item[kAsideOp]);
+                    n = uni(item[kAsideRows]);
+                    base = n >> 16;
+                    n &= 0xffffu;
+                    left = uni(item[kAsideLeft]);
+                    // the table's rows in shares for the waves
+                    const uint32_t share = max(kRGive, (n + (blockDim.x >> 6) - 1) / (blockDim.x >> 6)), first = t * share;
+                    if (first >= n) continue;
+                    n = min(share, n - first);
+                    const uint32_t at = V.wv + uni(item[kAsideCol]), cols = uni(item[kAsideCols]);
+                    const uint16_t* from = reinterpret_cast<const uint16_t*>(item + kRAside) + first;
+                    for (uint32_t k = 0; k < cols; ++k)
+                        for (uint32_t i = lane; i < n; i += 64) st16(at + k * kRCol + 2 * i, from[kRCap * k + i]);
+                } else {
+                    RTask task;
+                    if constexpr (kSmall) task = RTask{0, a.label0, 64 * t, 64, kNone, 0, 1, 0};
+                    else task = {tasks[t].op, tasks[t].label, tasks[t].first, tasks[t].rows, tasks[t].child, tasks[t].nchild, tasks[t].account, 0};
+                    opo = task.op;
+                    child = vec(task.child);
+                    nchild = vec(task.nchild);
+                    account = task.account;
+                    const uint32_t s0 = uni(ld16(o_lvo + 2 * task.label)) + task.first, s1 = uni(ld16(o_lvo + 2 * task.label + 2));
+                    if (s0 >= s1) continue;
+                    n = s1 - s0 < task.rows ? s1 - s0 : task.rows;
+                    for (uint32_t i = lane; i < n; i += 64) st16(V.wv + 2 * i, ld16(o_lv + 2 * (s0 + i)));
+                }
                 wave_lds_sync();
             } else {
                 // Wait for a share.  A giver counts itself and the taker as at
@@ -384,7 +458,7 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                     const uint32_t L0 = op.cols & 0xffffu, nleaf = op.cols >> 16;
                     for (uint32_t r0 = 0; r0 < n; r0 += 64) {
                         const uint32_t r = r0 + lane < n ? r0 + lane : r0;
-                        uint64_t by, c = rleaf_count(V, lf, leaf_cols, L0, nleaf, r, by);
+                        uint64_t by, c = rleaf_count(V, lf, (const GV_CONST uint32_t*)(ops + rargs().o_col), L0, nleaf, r, by);
                         if (r0 + lane >= n) c = by = 0;
                         sum0 += by;
                         sum1 += c;
@@ -429,6 +503,7 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                         if (__ballot(len != 0) == 0) continue;
                         const uint32_t incl = wave_scan_u32(len), excl = incl - len;
                         const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+                        spare = vec(spare - 1 - total / 64);
                         for (; c0 < total; c0 += 64) {
                             if (extend && nn > kRCap - 64) {
                                 suspended = 2;
@@ -504,17 +579,56 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                 if (lane < 2 && (w > 1 || account))
                     add64(o_acc + 16 * (head >> 16) + 8 * lane, lane ? sum1 : sum0);
                 cb = cc = 0;
+                bool aside = false;
                 if (nn) {
                     // down to the operations on the new table
                     wave_lds_sync();
                     opo = op.child;
                     if (!kSmall && w == 1) {
-                        opo = child;
-                        left = nchild;
+                        opo = uni(child);
+                        left = uni(nchild);
                     }
                     n = nn;
                     ++w;
                     if (n >= kRGive) {
+                        // (a table whose next operation only counts is soon done)
+                        if ((int)uni(spare) < 0 && (((const GV_CONST ROp*)(ops + opo))->head & 3u) == kOpExtend) {
+                            const GV_CONST RArgs& b = rargs();
+                            // while there are blocks to take no workgroup is idle,
+                            // and a tail soon over does not pay for a launch
+                            bool idle = true;
+                            if constexpr (!kSmall) {
+                                uint32_t at = 0;
+                                if (lane == 0) at = __hip_atomic_load(b.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                const bool none = uni(at) + gridDim.x >= b.nwork;
+                                idle = none && uni(tail);
+                                tail = vec(none);
+                                spare = vec(none ? kRTail : kRAgain);
+                            }
+                            uint32_t at = 0;
+                            if (idle) {
+                                if (lane == 0) at = atomicAdd(b.naside, 1u);
+                                at = uni(at);
+                                aside = at < b.aside_cap;
+                                spare = vec(aside ? 0xffffffffu : kRAgain);
+                            }
+                            if (aside) {
+                                uint32_t* to = b.aside + (uint64_t)at * b.item_words;
+                                const uint32_t cols = ((head >> 10) & 15u) + (op.cols >> 16 != kNoCol);
+                                if (lane == 0) {
+                                    to[kAsideBlock] = kAside ? b.items[(uint64_t)uni(wv) * b.item_words + kAsideBlock] : uni(wv);
+                                    to[kAsideOp] = opo;
+                                    to[kAsideRows] = n | w << 16;
+                                    to[kAsideLeft] = left;
+                                    to[kAsideCol] = op.dst;
+                                    to[kAsideCols] = cols;
+                                }
+                                for (uint32_t k = 0; k < cols; ++k)
+                                    to[kRAside + 64 * k + lane] = ld32(V.wv + op.dst + k * kRCol + 4 * lane);
+                            }
+                        }
+                    }
+                    if (!aside && n >= kRGive) {
                         // half of the rows to a wave that has nothing to do
                         const uint32_t idle = uni(ld32_shared(o_ctl + kCtlIdle));
                         if (idle) {
@@ -544,11 +658,11 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                             }
                         }
                     }
-                    continue;
+                    if (!aside) continue;
                 }
                 // the next operation on this table, or back up to the
                 // narrowest table that has work left
-                uint32_t nx = w == 1 || (!kSmall && w == 2 && --left == 0) ? kNone : op.next;
+                uint32_t nx = aside || w == 1 || (!kSmall && w == 2 && --left == 0) ? kNone : op.next;
                 while (nx == kNone && w > base) {
                     --w;
                     const uint32_t s = o_st + 16 * w;
@@ -568,10 +682,13 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                 opo = nx;
             }
         }
-        if (!kSmall && threadIdx.x == 0) st32(o_ctl + kCtlNext, then);
+        if (counter && threadIdx.x == 0) st32(o_ctl + kCtlNext, then);
         __syncthreads();
-        bi = gridDim.x + (kSmall ? bi : uni(ld32(o_ctl + kCtlNext)));
+        const uint32_t wnext = gridDim.x + (counter ? uni(ld32(o_ctl + kCtlNext)) : uni(wv));
         if (a.bits) {
+            // (read again: they are not worth registers while the block is mined)
+            const GV_CONST RArgs& a = rargs();
+            const RBlk& blk = a.blk[kAside ? a.items[(uint64_t)uni(wv) * a.item_words] : uni(wv)];
             for (uint32_t i = threadIdx.x; i < a.nterms * blk.gwords; i += blockDim.x) {
                 const uint32_t term = i / blk.gwords, x = i - term * blk.gwords;
                 const uint32_t o = o_bits + 4 * (term * a.gw + x);
@@ -582,6 +699,7 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                 }
             }
         }
+        wi = wnext;
         __syncthreads();
     }
     for (uint32_t i = threadIdx.x; i < 2 * a.nops; i += blockDim.x) {
@@ -591,11 +709,19 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
 }
 
 // The accumulators (their copies added up) and bitsets into pinned host
-// memory, cleared for the next launch.
+// memory, cleared for the next launch; or, when the launch set tables aside,
+// only their number (naside[which]).
 __global__ __launch_bounds__(256) void k_resident_out(unsigned long long* acc, uint32_t nacc, unsigned long long* hacc,
-                                                      uint32_t* next, uint32_t* bits, uint64_t nbits, uint32_t* hbits) {
+                                                      uint32_t* next, uint32_t* bits, uint64_t nbits, uint32_t* hbits,
+                                                      uint32_t* naside, uint32_t which, uint32_t* haside) {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
-    if (t == 0) *next = 0;
+    const uint32_t left = naside[which];
+    if (t == 0) {
+        *next = 0;
+        *haside = left;
+        naside[which ^ 1] = 0;   // those have been taken up
+    }
+    if (left) return;
     for (uint64_t i = t; i < nacc; i += stride) {
         uint64_t x = 0;
 #pragma unroll
@@ -873,20 +999,26 @@ int res_image_build(gv_graph* g, const uint32_t* graph_of) {
     HIPCHK(hipGetLastError());
     HIPCHK(hipDeviceSynchronize());
     const int most = kRLdsMost;
-    HIPCHK(hipFuncSetAttribute((const void*)k_resident<true>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
-    HIPCHK(hipFuncSetAttribute((const void*)k_resident<false>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    for (const auto kernel : {k_resident<true, false>, k_resident<false, false>, k_resident<true, true>, k_resident<false, true>})
+        HIPCHK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return GV_OK;
 }
 
 // ---- programs and calls ----------------------------------------------------
+
+constexpr uint64_t kRAccBytes = 16ull * kRMaxOps * kRLines;
+enum { kTailNext = 0, kTailAside = 1 };          // words: blocks handed out, tables set aside (two, in turn)
+constexpr uint64_t kRTailBytes = 16;
 
 // A context's buffers of gv_resident_mine, kept between calls (grow only).
 struct ResWork {
     char* d_prog = nullptr;               // operations, leaf descriptors, roots
     char* h_prog = nullptr;               // pinned
     uint64_t prog_cap = 0;
-    unsigned long long* d_acc = nullptr;  // kRLines copies of 2 kRMaxOps words, zero between calls
-    unsigned long long* h_acc = nullptr;  // pinned
+    // kRLines copies of 2 kRMaxOps words, the counters (kTail...), zero between
+    // calls; then twice kRAsideBytes of tables set aside
+    unsigned long long* d_acc = nullptr;
+    unsigned long long* h_acc = nullptr;  // pinned: 2 kRMaxOps words and the number set aside
     uint32_t* d_bits = nullptr;           // zero between calls
     uint32_t* h_bits = nullptr;           // pinned
     uint64_t bits_cap = 0;
@@ -920,9 +1052,9 @@ struct RProg {
         uint32_t live = 0;                // columns kept
         uint32_t off = 0;                 // where, in a wave's levels
         double rows = 0;                  // expected in a block
-        std::vector<uint32_t> labels;     // of its columns
     };
     const gv_graph* g;
+    double nblk;                          // blocks of the database
     std::vector<Op> ops;
     std::vector<Table> tables;
     std::map<uint32_t, uint32_t> start;   // label -> its start table
@@ -932,9 +1064,10 @@ struct RProg {
     std::vector<RLeafStep> leaves;
     std::vector<uint32_t> cols;           // same-label columns of leaf steps
     std::vector<RTask> tasks;
-    uint32_t lvl_bytes = 0, nroots = 0;
+    uint32_t lvl_bytes = 0, nroots = 0, most_cols = 1;
+    double all_rows = 0;                  // that operations read and make, expected in a block
 
-    explicit RProg(const gv_graph* g_) : g(g_) {}
+    RProg(const gv_graph* g_, uint32_t blocks) : g(g_), nblk(blocks) {}
 
     static bool same(const gv_step_t& x, const gv_step_t& y) {
         return x.label == y.label && x.nback == y.nback && x.ncoll == y.ncoll && x.restrict_col == y.restrict_col &&
@@ -954,14 +1087,28 @@ struct RProg {
         }
         return true;
     }
-    uint32_t table(uint32_t width, uint32_t label0, uint32_t from) {
+    uint32_t table(uint32_t width, uint32_t label0, uint32_t from, double rows) {
         Table t;
         t.width = width;
         t.label0 = label0;
         t.from = from;
+        t.rows = rows;
         tables.push_back(t);
         lmax = std::max(lmax, width);
         return (uint32_t)tables.size() - 1;
+    }
+
+    double vertices(uint32_t label) const { return (double)(g->lvoff[label + 1] - g->lvoff[label]); }
+    // Rows that step w of a query makes of one row, from the label statistics.
+    double growth(const gv_query_t& q, uint32_t w) const {
+        const gv_step_t& s = q.step[w];
+        const uint64_t nl = g->nlabels;
+        double f = 1e300;
+        for (uint32_t i = 0; i < s.nback; ++i) {
+            const uint64_t l = s.back_col[i] ? q.step[s.back_col[i]].label : q.label0;
+            f = std::min(f, (double)g->pair_edges[(s.back_part[i] * nl + l) * nl + s.label] / std::max(1.0, vertices((uint32_t)l)));
+        }
+        return f;
     }
 
     // Adds a query's operations; `path` receives them from the start table
@@ -969,7 +1116,7 @@ struct RProg {
     bool add(const gv_query_t& q, const gv_leaves_t* lv, std::vector<uint32_t>& path) {
         bool reused = false;
         auto it = start.find(q.label0);
-        if (it == start.end()) it = start.emplace(q.label0, table(1, q.label0, kNone)).first;
+        if (it == start.end()) it = start.emplace(q.label0, table(1, q.label0, kNone, vertices(q.label0) / nblk)).first;
         uint32_t t = it->second;
         for (uint32_t w = 1;; ++w) {
             const bool leafy = lv && w == lv->width, end = leafy || w + 1 == q.k;
@@ -988,8 +1135,12 @@ struct RProg {
                 } else {
                     o.st = q.step[w];
                 }
+                // (the hubs that many rows run through have more neighbours than the mean)
+                const double rows = tables[t].rows,
+                             made = leafy ? 0.0 : rows * growth(q, w) * (q.step[w].nback > 1 ? 0.2 : 1.5);
+                all_rows += rows + made;
                 if (end) o.term = nterms++;
-                else o.child = table(w + 1, q.label0, id);
+                else o.child = table(w + 1, q.label0, id, made);
                 ops.push_back(o);
                 tables[t].ops.push_back(id);
             } else if (w == 1) {
@@ -1032,6 +1183,7 @@ struct RProg {
                 t.live = 1;
             }
             lvl_bytes = std::max(lvl_bytes, t.off + kRCol * (uint32_t)__builtin_popcount(t.live));
+            most_cols = std::max(most_cols, (uint32_t)__builtin_popcount(t.live));
         }
         auto col = [&](const Table& t, uint32_t c) {
             return t.off + kRCol * (uint32_t)__builtin_popcount(t.live & ((1u << c) - 1));
@@ -1134,30 +1286,8 @@ struct RProg {
 // 1 / kRShares of the block's expected work (from the label statistics), and
 // at most kRCap.  Heavy shares go first.
 void make_tasks(RProg& p, const ResImage* R) {
-    const gv_graph* g = p.g;
-    const uint32_t nl = g->nlabels, n = (uint32_t)p.ops.size();
+    const uint32_t n = (uint32_t)p.ops.size();
     std::vector<double> cost(n, 0);   // batches of an operation and of those below it, in a block
-    for (uint32_t t = 0; t < p.tables.size(); ++t) {
-        RProg::Table& T = p.tables[t];
-        if (T.from == kNone) {
-            T.labels.assign(1, T.label0);
-            T.rows = (double)(g->lvoff[T.label0 + 1] - g->lvoff[T.label0]) / R->nblk;
-        } else {
-            const RProg::Op& o = p.ops[T.from];
-            const RProg::Table& U = p.tables[o.table];
-            double f = 1e300;
-            for (uint32_t i = 0; i < o.st.nback; ++i) {
-                const uint64_t l = U.labels[o.st.back_col[i]], nv = g->lvoff[l + 1] - g->lvoff[l];
-                f = std::min(f, (double)g->pair_edges[(o.st.back_part[i] * (uint64_t)nl + l) * nl + o.st.label] /
-                                    std::max<double>(1.0, (double)nv));
-            }
-            T.labels = U.labels;
-            T.labels.push_back(o.st.label);
-            T.rows = U.rows * f;
-            // the hubs that many rows run through have more neighbours than the mean
-            T.rows *= o.st.nback > 1 ? 0.2 : 1.5;
-        }
-    }
     for (uint32_t x = n; x-- > 0;) {
         const RProg::Op& o = p.ops[x];
         cost[x] += 1.0 + p.tables[o.table].rows / 64 * (o.kind == kOpLeaves ? 1.0 : 2.0);
@@ -1215,13 +1345,13 @@ int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
     // (each of the two on its own: a call that found memory for one of them
     // only leaves that one for the next)
     if (!w->d_acc) {
-        if (hipMalloc(&w->d_acc, 16 * kRMaxOps * kRLines + 16) != hipSuccess) {
+        if (hipMalloc(&w->d_acc, kRAccBytes + kRTailBytes + 2 * kRAsideBytes) != hipSuccess) {
             w->d_acc = nullptr;
             return GV_ERR_NOMEM;
         }
         w->dirty = true;
     }
-    if (!w->h_acc && hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps, hipHostMallocCoherent) != hipSuccess) {
+    if (!w->h_acc && hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps + 16, hipHostMallocCoherent) != hipSuccess) {
         w->h_acc = nullptr;
         return GV_ERR_NOMEM;
     }
@@ -1249,7 +1379,7 @@ int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
         w->dirty = true;
     }
     if (w->dirty) {
-        HIPCHK(hipMemsetAsync(w->d_acc, 0, 16 * kRMaxOps * kRLines + 16, c->stream));
+        HIPCHK(hipMemsetAsync(w->d_acc, 0, kRAccBytes + kRTailBytes, c->stream));
         if (w->d_bits) HIPCHK(hipMemsetAsync(w->d_bits, 0, 4 * w->bits_cap, c->stream));
         w->dirty = false;
     }
@@ -1274,7 +1404,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
     std::vector<std::vector<uint32_t>> paths;
     for (uint32_t i0 = 0; i0 < n;) {
         // as many queries as one launch takes
-        RProg p(g);
+        RProg p(g, R->nblk);
         uint32_t i1 = i0;
         paths.clear();
         while (i1 < n && p.ops.size() + qs[i1]->k <= kRMaxOps && p.nterms < kRMaxTerms) {
@@ -1300,7 +1430,6 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         RArgs a;
         a.blk = R->d_blk;
         a.img = R->d_img;
-        a.nblk = R->nblk;
         a.mask_words = R->mask_words;
         a.ops = nullptr;
         a.tasks = nullptr;
@@ -1315,7 +1444,13 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         a.img_bytes = R->img_bytes;
         a.nwords = nwords;
         a.acc = w->d_acc;
-        a.next = reinterpret_cast<uint32_t*>(w->d_acc + 2 * kRMaxOps * kRLines);
+        uint32_t* const tail = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(w->d_acc) + kRAccBytes);
+        uint32_t* const aside[2] = {tail + kRTailBytes / 4, tail + (kRTailBytes + kRAsideBytes) / 4};
+        uint32_t* const left = reinterpret_cast<uint32_t*>(w->h_acc + 2 * kRMaxOps);
+        a.next = tail + kTailNext;
+        a.nwork = R->nblk;
+        a.item_words = kRAside + 64 * p.most_cols;
+        a.aside_cap = (uint32_t)(kRAsideBytes / 4 / a.item_words);
         a.bits = bits ? w->d_bits : nullptr;
         if (small) {
             p.image(reinterpret_cast<char*>(a.prog));
@@ -1349,20 +1484,34 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         const uint32_t lds = fixed + waves * each;
         if (waves == 0 || lds > kRLdsMost) return GV_ERR_CAPACITY;
         const uint32_t per_cu = std::max<uint32_t>(1, std::min<uint32_t>(kRLdsMost / lds, 32 / waves));
-        const uint32_t grid = std::min<uint32_t>(R->nblk, per_cu * c->num_cu);
+        // the expected mean over the waves of the chip, or of all blocks' if those are more
+        const uint32_t groups = std::max(R->nblk, per_cu * (uint32_t)c->num_cu);
+        a.budget = (uint32_t)std::min(1e9, kRSpare + p.all_rows * R->nblk / (64.0 * waves * groups));
         w->dirty = true;
-        {
-            ProfScope ps(c, kKindResident);
-            if (small) hipLaunchKernelGGL(k_resident<true>, dim3(grid), dim3(64 * waves), lds, c->stream, a);
-            else hipLaunchKernelGGL(k_resident<false>, dim3(grid), dim3(64 * waves), lds, c->stream, a);
+        for (uint32_t turn = 0;; ++turn) {
+            a.aside = aside[turn & 1];
+            a.naside = tail + kTailAside + (turn & 1);
+            *left = 0;
+            {
+                ProfScope ps(c, kKindResident);
+                const uint32_t grid = std::min<uint32_t>(a.nwork, per_cu * c->num_cu);
+                const auto kernel = turn ? (small ? k_resident<true, true> : k_resident<false, true>)
+                                         : (small ? k_resident<true, false> : k_resident<false, false>);
+                hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * waves), lds, c->stream, a);
+                HIPCHK(hipGetLastError());
+            }
+            hipLaunchKernelGGL(k_resident_out, dim3(grid_for(std::max<uint64_t>(nb, 2 * nops), 256, 512)), dim3(256), 0,
+                               c->stream, w->d_acc, 2 * nops, w->h_acc, a.next, w->d_bits, nb, w->h_bits,
+                               tail + kTailAside, turn & 1, left);
             HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(c->stream));
+            st.launches += 1;
+            if (*left == 0) break;
+            // the tables that were set aside, over the whole chip
+            a.items = a.aside;
+            a.nwork = std::min<uint32_t>(*left, a.aside_cap);
         }
-        hipLaunchKernelGGL(k_resident_out, dim3(grid_for(std::max<uint64_t>(nb, 2 * nops), 256, 512)), dim3(256), 0,
-                           c->stream, w->d_acc, 2 * nops, w->h_acc, a.next, w->d_bits, nb, w->h_bits);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(c->stream));
         w->dirty = false;
-        st.launches += 1;
         // bytes of each operation from the rows it read, its lists and what it wrote
         std::vector<uint64_t> by(nops);
         for (uint32_t x = 0; x < nops; ++x) {
