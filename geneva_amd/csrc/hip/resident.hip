@@ -133,7 +133,8 @@ struct RArgs {
     uint32_t* aside;             // for the next launch: `naside` of at most aside_cap
     uint32_t* naside;
     uint32_t aside_cap;
-    uint32_t budget;             // batches a wave works through in a block before it sets tables aside (below 2^31)
+    uint32_t busy;               // set aside with so many workgroups at work, or fewer
+    uint32_t* done;              // workgroups that have ended: kRLines counters, kRDoneStep words apart
     uint32_t* bits;              // nterms x nwords (nullable)
     uint32_t prog[kRSmallBytes / 4];   // a small program
 };
@@ -148,24 +149,25 @@ constexpr uint32_t kRLdsMost = 160u << 10;       // LDS of a CU
 constexpr uint32_t kRSmallWaves = 4, kRWaves = 8;   // waves of a workgroup, at most
 constexpr uint32_t kRGive = 16;                  // rows of a table worth sharing; 4 or 48: within 2%
 constexpr uint64_t kRAsideBytes = 4u << 20;      // tables set aside by one launch, at most
-// A wave's work in a block, in batches of 64 rows and of 64 candidates, before
-// it sets tables aside: kRSpare (about 80 us of a wave alone) and the mean over
-// the waves that the label statistics let expect.  The blocks of a batch are
-// handed out one by one, so there it first looks again every kRAgain whether
-// any is left, and works through kRTail after the last.  What is set aside
-// costs another launch and a synchronisation (35 us) and its block's image
-// again.  Calls on databases with hubs, without and with it, and with the
-// table engines:
-//   a star query on 6,000 graphs of 20-400 vertices       1330 ->  342 us  ( 285)
-//   200 queries on the same, one call                     3.21 -> 1.76 ms  (3.48)
-//   9 queries on 8 graphs of 1,450 vertices, one by one   1746 ->  933 us  (1448)
-//   9 on 20,000 small and 10 such graphs, one by one      2589 -> 1024 us  (2637)
+// A wave sets tables aside once it has worked through kRSpare batches of 64
+// rows or 64 candidates in a block (about 80 us alone), while a quarter of the
+// workgroups that the chip holds or fewer are at work; it looks again every
+// kRAgain.  What is set aside costs another launch and a synchronisation (35
+// us) and its block's image again, so it does not pay while the chip is busy
+// (9 queries on 5,000 hub graphs, heavy in every block: 2008 us with nothing
+// set aside, 2085 without this condition, 1857 with it).  Calls on databases
+// with hubs, without and with it, and with the table engines:
+//   a star query on 6,000 graphs of 20-400 vertices       1380 ->  341 us  ( 289)
+//   131 queries on the same, one call                     3.02 -> 1.56 ms  (2.89)
+//   9 queries on 8 graphs of 1,450 vertices, one by one   1684 -> 1038 us  (1448)
+//   the same, one call                                     867 ->  329 us  ( 588)
+//   9 on 20,000 small and 10 such graphs, one by one      2467 -> 1048 us  (2637)
 // 600 queries, one by one, on two databases without such hubs: the sum within
-// 1%, on one with them 6% less; batches of 24 to 600 of them 3% more to 43%
-// less.  With kRSpare 100 / 200 / 300 the heaviest of the 600 took 472 / 548 /
-// 602 us; without kRTail batches that end evenly were up to 10% slower.
-constexpr double kRSpare = 160;
-constexpr uint32_t kRTail = 256, kRAgain = 64;
+// 1%, on one with them 5% less; batches of 24 to 600 of them between 7% more
+// (600 us) and 48% less.  kRSpare 100: the sums 0-1% more, the heaviest 10%
+// less; half or an eighth of the workgroups: within 5%.
+constexpr uint32_t kRSpare = 160, kRAgain = 64;
+constexpr uint32_t kRDoneStep = 16;              // words: a cache line
 // a workgroup's control words: tasks taken, next block, waves waiting for a
 // share (a bit each), waves at work; then each wave's share: given | first
 // operation | rows, width << 16 | operations left on a width-2 table
@@ -373,8 +375,7 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
         V.nbr = V.doff + 2 * (blk.ndir + 1);
         const uint32_t o_lv = V.nbr + 2 * blk.ne, o_lvo = o_lv + 2 * blk.nv;
         __syncthreads();
-        uint32_t spare = vec(a.budget);   // batches before this wave sets tables aside (as int)
-        uint32_t tail = vec(0);           // whether no block was left when it last looked
+        uint32_t spare = vec(kRSpare);    // batches before this wave sets tables aside (as int)
         bool drained = false;   // no task is left: this wave takes shares of the others' work
         for (;;) {
             uint32_t opo, n;              // the operation, and rows of the table it reads
@@ -594,24 +595,13 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
                         // (a table whose next operation only counts is soon done)
                         if ((int)uni(spare) < 0 && (((const GV_CONST ROp*)(ops + opo))->head & 3u) == kOpExtend) {
                             const GV_CONST RArgs& b = rargs();
-                            // while there are blocks to take no workgroup is idle,
-                            // and a tail soon over does not pay for a launch
-                            bool idle = true;
-                            if constexpr (!kSmall) {
-                                uint32_t at = 0;
-                                if (lane == 0) at = __hip_atomic_load(b.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                const bool none = uni(at) + gridDim.x >= b.nwork;
-                                idle = none && uni(tail);
-                                tail = vec(none);
-                                spare = vec(none ? kRTail : kRAgain);
-                            }
-                            uint32_t at = 0;
-                            if (idle) {
-                                if (lane == 0) at = atomicAdd(b.naside, 1u);
-                                at = uni(at);
-                                aside = at < b.aside_cap;
-                                spare = vec(aside ? 0xffffffffu : kRAgain);
-                            }
+                            uint32_t ended = 0;
+                            if (lane < kRLines) ended = __hip_atomic_load(b.done + kRDoneStep * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            uint32_t at = b.aside_cap;
+                            if (gridDim.x - wave_total_u32(ended) <= b.busy && lane == 0) at = atomicAdd(b.naside, 1u);
+                            at = uni(at);
+                            aside = at < b.aside_cap;
+                            spare = vec(aside ? 0xffffffffu : kRAgain);
                             if (aside) {
                                 uint32_t* to = b.aside + (uint64_t)at * b.item_words;
                                 const uint32_t cols = ((head >> 10) & 15u) + (op.cols >> 16 != kNoCol);
@@ -702,6 +692,7 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
         wi = wnext;
         __syncthreads();
     }
+    if (threadIdx.x == 0) atomicAdd(a.done + kRDoneStep * (blockIdx.x % kRLines), 1u);
     for (uint32_t i = threadIdx.x; i < 2 * a.nops; i += blockDim.x) {
         const uint64_t x = *reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(rlds) + o_acc + 8 * i);
         if (x) atomicAdd(&a.acc[(blockIdx.x % kRLines) * 2 * a.nops + i], (unsigned long long)x);
@@ -713,27 +704,38 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
 // only their number (naside[which]).
 __global__ __launch_bounds__(256) void k_resident_out(unsigned long long* acc, uint32_t nacc, unsigned long long* hacc,
                                                       uint32_t* next, uint32_t* bits, uint64_t nbits, uint32_t* hbits,
-                                                      uint32_t* naside, uint32_t which, uint32_t* haside) {
+                                                      uint32_t* naside, uint32_t which, uint32_t* haside, uint32_t* done) {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    // the first of each thread's words are on their way before `left` is known
     const uint32_t left = naside[which];
+    uint64_t x = 0;
+    uint32_t m = 0;
+    if (t < nacc)
+#pragma unroll
+        for (uint32_t k = 0; k < kRLines; ++k) x += acc[k * nacc + t];
+    if (t < nbits) m = bits[t];
     if (t == 0) {
         *next = 0;
         *haside = left;
         naside[which ^ 1] = 0;   // those have been taken up
     }
+    if (t < kRLines) done[kRDoneStep * t] = 0;
     if (left) return;
-    for (uint64_t i = t; i < nacc; i += stride) {
-        uint64_t x = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < kRLines; ++k) {
-            x += acc[k * nacc + i];
-            acc[k * nacc + i] = 0;
-        }
+    for (uint64_t i = t; i < nacc;) {
         hacc[i] = x;
+#pragma unroll
+        for (uint32_t k = 0; k < kRLines; ++k) acc[k * nacc + i] = 0;
+        i += stride;
+        x = 0;
+        if (i < nacc)
+#pragma unroll
+            for (uint32_t k = 0; k < kRLines; ++k) x += acc[k * nacc + i];
     }
-    for (uint64_t i = t; i < nbits; i += stride) {
-        hbits[i] = bits[i];
+    for (uint64_t i = t; i < nbits;) {
+        hbits[i] = m;
         bits[i] = 0;
+        i += stride;
+        if (i < nbits) m = bits[i];
     }
 }
 
@@ -1007,8 +1009,9 @@ int res_image_build(gv_graph* g, const uint32_t* graph_of) {
 // ---- programs and calls ----------------------------------------------------
 
 constexpr uint64_t kRAccBytes = 16ull * kRMaxOps * kRLines;
-enum { kTailNext = 0, kTailAside = 1 };          // words: blocks handed out, tables set aside (two, in turn)
-constexpr uint64_t kRTailBytes = 16;
+// words: blocks handed out, tables set aside (two, in turn), workgroups that ended
+enum { kTailNext = 0, kTailAside = 1, kTailDone = kRDoneStep };
+constexpr uint64_t kRTailBytes = 4 * kRDoneStep * (1 + kRLines);
 
 // A context's buffers of gv_resident_mine, kept between calls (grow only).
 struct ResWork {
@@ -1052,9 +1055,9 @@ struct RProg {
         uint32_t live = 0;                // columns kept
         uint32_t off = 0;                 // where, in a wave's levels
         double rows = 0;                  // expected in a block
+        std::vector<uint32_t> labels;     // of its columns
     };
     const gv_graph* g;
-    double nblk;                          // blocks of the database
     std::vector<Op> ops;
     std::vector<Table> tables;
     std::map<uint32_t, uint32_t> start;   // label -> its start table
@@ -1065,9 +1068,8 @@ struct RProg {
     std::vector<uint32_t> cols;           // same-label columns of leaf steps
     std::vector<RTask> tasks;
     uint32_t lvl_bytes = 0, nroots = 0, most_cols = 1;
-    double all_rows = 0;                  // that operations read and make, expected in a block
 
-    RProg(const gv_graph* g_, uint32_t blocks) : g(g_), nblk(blocks) {}
+    explicit RProg(const gv_graph* g_) : g(g_) {}
 
     static bool same(const gv_step_t& x, const gv_step_t& y) {
         return x.label == y.label && x.nback == y.nback && x.ncoll == y.ncoll && x.restrict_col == y.restrict_col &&
@@ -1087,28 +1089,14 @@ struct RProg {
         }
         return true;
     }
-    uint32_t table(uint32_t width, uint32_t label0, uint32_t from, double rows) {
+    uint32_t table(uint32_t width, uint32_t label0, uint32_t from) {
         Table t;
         t.width = width;
         t.label0 = label0;
         t.from = from;
-        t.rows = rows;
         tables.push_back(t);
         lmax = std::max(lmax, width);
         return (uint32_t)tables.size() - 1;
-    }
-
-    double vertices(uint32_t label) const { return (double)(g->lvoff[label + 1] - g->lvoff[label]); }
-    // Rows that step w of a query makes of one row, from the label statistics.
-    double growth(const gv_query_t& q, uint32_t w) const {
-        const gv_step_t& s = q.step[w];
-        const uint64_t nl = g->nlabels;
-        double f = 1e300;
-        for (uint32_t i = 0; i < s.nback; ++i) {
-            const uint64_t l = s.back_col[i] ? q.step[s.back_col[i]].label : q.label0;
-            f = std::min(f, (double)g->pair_edges[(s.back_part[i] * nl + l) * nl + s.label] / std::max(1.0, vertices((uint32_t)l)));
-        }
-        return f;
     }
 
     // Adds a query's operations; `path` receives them from the start table
@@ -1116,7 +1104,7 @@ struct RProg {
     bool add(const gv_query_t& q, const gv_leaves_t* lv, std::vector<uint32_t>& path) {
         bool reused = false;
         auto it = start.find(q.label0);
-        if (it == start.end()) it = start.emplace(q.label0, table(1, q.label0, kNone, vertices(q.label0) / nblk)).first;
+        if (it == start.end()) it = start.emplace(q.label0, table(1, q.label0, kNone)).first;
         uint32_t t = it->second;
         for (uint32_t w = 1;; ++w) {
             const bool leafy = lv && w == lv->width, end = leafy || w + 1 == q.k;
@@ -1135,12 +1123,8 @@ struct RProg {
                 } else {
                     o.st = q.step[w];
                 }
-                // (the hubs that many rows run through have more neighbours than the mean)
-                const double rows = tables[t].rows,
-                             made = leafy ? 0.0 : rows * growth(q, w) * (q.step[w].nback > 1 ? 0.2 : 1.5);
-                all_rows += rows + made;
                 if (end) o.term = nterms++;
-                else o.child = table(w + 1, q.label0, id, made);
+                else o.child = table(w + 1, q.label0, id);
                 ops.push_back(o);
                 tables[t].ops.push_back(id);
             } else if (w == 1) {
@@ -1286,8 +1270,30 @@ struct RProg {
 // 1 / kRShares of the block's expected work (from the label statistics), and
 // at most kRCap.  Heavy shares go first.
 void make_tasks(RProg& p, const ResImage* R) {
-    const uint32_t n = (uint32_t)p.ops.size();
+    const gv_graph* g = p.g;
+    const uint32_t nl = g->nlabels, n = (uint32_t)p.ops.size();
     std::vector<double> cost(n, 0);   // batches of an operation and of those below it, in a block
+    for (uint32_t t = 0; t < p.tables.size(); ++t) {
+        RProg::Table& T = p.tables[t];
+        if (T.from == kNone) {
+            T.labels.assign(1, T.label0);
+            T.rows = (double)(g->lvoff[T.label0 + 1] - g->lvoff[T.label0]) / R->nblk;
+        } else {
+            const RProg::Op& o = p.ops[T.from];
+            const RProg::Table& U = p.tables[o.table];
+            double f = 1e300;
+            for (uint32_t i = 0; i < o.st.nback; ++i) {
+                const uint64_t l = U.labels[o.st.back_col[i]], nv = g->lvoff[l + 1] - g->lvoff[l];
+                f = std::min(f, (double)g->pair_edges[(o.st.back_part[i] * (uint64_t)nl + l) * nl + o.st.label] /
+                                    std::max<double>(1.0, (double)nv));
+            }
+            T.labels = U.labels;
+            T.labels.push_back(o.st.label);
+            T.rows = U.rows * f;
+            // the hubs that many rows run through have more neighbours than the mean
+            T.rows *= o.st.nback > 1 ? 0.2 : 1.5;
+        }
+    }
     for (uint32_t x = n; x-- > 0;) {
         const RProg::Op& o = p.ops[x];
         cost[x] += 1.0 + p.tables[o.table].rows / 64 * (o.kind == kOpLeaves ? 1.0 : 2.0);
@@ -1404,7 +1410,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
     std::vector<std::vector<uint32_t>> paths;
     for (uint32_t i0 = 0; i0 < n;) {
         // as many queries as one launch takes
-        RProg p(g, R->nblk);
+        RProg p(g);
         uint32_t i1 = i0;
         paths.clear();
         while (i1 < n && p.ops.size() + qs[i1]->k <= kRMaxOps && p.nterms < kRMaxTerms) {
@@ -1448,6 +1454,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         uint32_t* const aside[2] = {tail + kRTailBytes / 4, tail + (kRTailBytes + kRAsideBytes) / 4};
         uint32_t* const left = reinterpret_cast<uint32_t*>(w->h_acc + 2 * kRMaxOps);
         a.next = tail + kTailNext;
+        a.done = tail + kTailDone;
         a.nwork = R->nblk;
         a.item_words = kRAside + 64 * p.most_cols;
         a.aside_cap = (uint32_t)(kRAsideBytes / 4 / a.item_words);
@@ -1484,9 +1491,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         const uint32_t lds = fixed + waves * each;
         if (waves == 0 || lds > kRLdsMost) return GV_ERR_CAPACITY;
         const uint32_t per_cu = std::max<uint32_t>(1, std::min<uint32_t>(kRLdsMost / lds, 32 / waves));
-        // the expected mean over the waves of the chip, or of all blocks' if those are more
-        const uint32_t groups = std::max(R->nblk, per_cu * (uint32_t)c->num_cu);
-        a.budget = (uint32_t)std::min(1e9, kRSpare + p.all_rows * R->nblk / (64.0 * waves * groups));
+        a.busy = per_cu * (uint32_t)c->num_cu / 4;
         w->dirty = true;
         for (uint32_t turn = 0;; ++turn) {
             a.aside = aside[turn & 1];
@@ -1502,7 +1507,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
             }
             hipLaunchKernelGGL(k_resident_out, dim3(grid_for(std::max<uint64_t>(nb, 2 * nops), 256, 512)), dim3(256), 0,
                                c->stream, w->d_acc, 2 * nops, w->h_acc, a.next, w->d_bits, nb, w->h_bits,
-                               tail + kTailAside, turn & 1, left);
+                               tail + kTailAside, turn & 1, left, a.done);
             HIPCHK(hipGetLastError());
             HIPCHK(hipStreamSynchronize(c->stream));
             st.launches += 1;
