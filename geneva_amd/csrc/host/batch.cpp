@@ -116,6 +116,7 @@ int BatchMiner::setPairStart(bool on) {
 }
 int BatchMiner::setProfile(bool on) {
     profile_ = on;
+    if (!on && !b_) return GV_OK;
     gv_batch_t b;
     int rc = engine(&b);
     return rc == GV_OK ? gv_batch_profile(b, on) : rc;

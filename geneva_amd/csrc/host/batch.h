@@ -54,6 +54,7 @@ public:
     // needed (a packed database mostly runs without it).
     int init();
     int engine(gv_batch_t* b);
+    gv_batch_t made() const { return b_; }   // the slot engine, null before that
     int setTune(const gv_tune_t& t);
     // Rows sized per iteration (at most options().rowCap, the allocation).
     int setRowCap(uint64_t rows);

@@ -673,9 +673,10 @@ int gh_engine_batch_profile(gh_engine_t e, int on) {
 
 int gh_engine_batch_profile_bytes(gh_engine_t e, uint64_t* size_bytes, uint64_t* walk_bytes) {
     if (!e || !e->batch) return GV_ERR_ARG;
-    gv_batch_t b;
-    int rc = e->batch->engine(&b);
-    return rc == GV_OK ? gv_batch_profile_bytes(b, size_bytes, walk_bytes) : rc;
+    if (e->batch->made()) return gv_batch_profile_bytes(e->batch->made(), size_bytes, walk_bytes);
+    if (size_bytes) *size_bytes = 0;
+    if (walk_bytes) *walk_bytes = 0;
+    return GV_OK;
 }
 
 int gh_engine_batch_pair_start(gh_engine_t e, int on) {
@@ -714,10 +715,10 @@ int gh_engine_batch_fused_rows(gh_engine_t e, uint64_t* rows) {
 }
 
 int gh_engine_batch_history(gh_engine_t e, uint64_t* rows, uint64_t* candidates, uint32_t cap, uint32_t* n) {
-    if (!e || !e->batch) return GV_ERR_ARG;
-    gv_batch_t b;
-    int rc = e->batch->engine(&b);
-    return rc == GV_OK ? gv_batch_history(b, rows, candidates, cap, n) : rc;
+    if (!e || !e->batch || !n) return GV_ERR_ARG;
+    if (e->batch->made()) return gv_batch_history(e->batch->made(), rows, candidates, cap, n);
+    *n = 0;
+    return GV_OK;
 }
 
 int gh_engine_profile_records(gh_engine_t e, int* kinds, float* ms, uint64_t cap, uint64_t* n) {

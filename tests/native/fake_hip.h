@@ -16,6 +16,7 @@
 namespace fake {
 inline int fail_alloc = -1;          // allocations until one fails (-1: none does)
 inline bool failed = false;          // that allocation was asked for
+inline int allocations = 0;          // device and pinned, so far
 inline bool sticky = false;          // a failed call is what hipGetLastError reports next
 inline hipError_t last = hipSuccess;
 inline int device = -1;              // of the last hipSetDevice
@@ -32,6 +33,7 @@ inline hipError_t alloc(void** p, size_t n) {
         if (sticky) last = hipErrorOutOfMemory;
         return hipErrorOutOfMemory;
     }
+    ++allocations;
     *p = std::malloc(n + 64);
     std::memset(*p, 0xab, n + 64);
     return hipSuccess;

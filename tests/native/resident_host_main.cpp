@@ -2,6 +2,7 @@
 // without a device: one case a run, named by the first argument.
 #include "fake_hip.h"
 #include "geneva_hip.h"
+#include "geneva_host.h"
 
 #include <new>
 
@@ -223,6 +224,34 @@ void no_host_memory() {
         }
 }
 
+// Reading the slot engine's counters, or turning its profile off, makes no
+// slot engine (device memory of slots x two tables) on a database that is
+// mined without it.
+void counters_without_slot_engine() {
+    fake::on_launch = pack_kernels;
+    const uint32_t labels[] = {0, 1, 2, 1, 2}, edges[] = {1, 2, 1, 3, 4, 1};
+    gh_dataset_t ds = gh_ds_from_arrays(4, labels, 2, edges, kOwner, 2);
+    CHECK(ds != nullptr);
+    int rc = 0;
+    gh_engine_t e = gh_engine_create(ds, 0, 1 << 20, &rc);
+    CHECK(e != nullptr && rc == GV_OK);
+    CHECK(gh_engine_resident_blocks(e) > 0);
+    CHECK(gh_engine_batch_config(e, 4, 1 << 20, 1 << 16, 0, 0) == GV_OK);
+    const char* q = "v 0 1\nv 1 2\ne 0 1 1\n";
+    uint64_t count = 0, bytes = 0;
+    uint32_t word = 0;
+    CHECK(gh_engine_batch_mine(e, &q, 1, 0, &count, &bytes, &word, 1, nullptr) == GV_OK);
+    const int held = fake::allocations;
+    CHECK(gh_engine_batch_profile(e, 0) == GV_OK);
+    uint64_t a = 1, b = 1, rows = 1, cand = 1;
+    CHECK(gh_engine_batch_profile_bytes(e, &a, &b) == GV_OK && a == 0 && b == 0);
+    uint32_t n = 1;
+    CHECK(gh_engine_batch_history(e, &rows, &cand, 1, &n) == GV_OK && n == 0);
+    CHECK(fake::allocations == held);
+    gh_engine_free(e);
+    gh_ds_free(ds);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -233,6 +262,7 @@ int main(int, char** argv) {
     else if (what == "owners_on_their_device") owners_on_their_device();
     else if (what == "packing_fails") packing_fails();
     else if (what == "no_host_memory") no_host_memory();
+    else if (what == "counters_without_slot_engine") counters_without_slot_engine();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;

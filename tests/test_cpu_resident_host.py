@@ -21,14 +21,15 @@ def exe(tmp_path_factory):
     lib = os.path.dirname(G.HIP_LIB)
     cmd = ["g++", "-std=c++17", "-O1", "-g", "-rdynamic", "-Wno-unused-result", "-I" + os.path.join(ROOT, "include"),
            "-I/opt/rocm/include", "-o", out, os.path.join(NATIVE, "resident_host_main.cpp"),
-           "-L" + lib, "-lgeneva_hip", "-Wl,-rpath," + lib, "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"]
+           "-L" + lib, "-lgeneva_host", "-lgeneva_hip", "-Wl,-rpath," + lib, "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
     return out
 
 
 @pytest.mark.parametrize("case", ["failed_allocation", "no_memory_is_capacity", "owners_twice",
-                                  "owners_on_their_device", "packing_fails", "no_host_memory"])
+                                  "owners_on_their_device", "packing_fails", "no_host_memory",
+                                  "counters_without_slot_engine"])
 def test_resident_host(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
