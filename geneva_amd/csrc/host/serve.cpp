@@ -173,8 +173,9 @@ static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
                 const int rc = direct(next);
                 if (rc != GV_OK) return rc;
             } else {
-                if (!now.empty() && inUse + est[next] > memBudget) break;
-                inUse += est[next];
+                // (estimates go up to 2^64 - 1: their sum may not)
+                if (!now.empty() && (inUse > memBudget || est[next] > memBudget - inUse)) break;
+                inUse = est[next] > UINT64_MAX - inUse ? UINT64_MAX : inUse + est[next];
                 now.push_back(next);
             }
         }

@@ -252,6 +252,55 @@ void counters_without_slot_engine() {
     gh_ds_free(ds);
 }
 
+// A packed database of two graphs: 60 vertices of label 1, all joined, and a
+// pair; path(k) is a path of k vertices of label 1.
+struct Served {
+    gh_dataset_t ds = nullptr;
+    gh_engine_t e = nullptr;
+    double stats[6] = {};
+    Served() {
+        std::vector<uint32_t> labels(63, 1), edges, owner(63, 0);
+        for (uint32_t a = 1; a <= 60; ++a)
+            for (uint32_t b = a + 1; b <= 60; ++b) edges.insert(edges.end(), {a, b, 1});
+        edges.insert(edges.end(), {61, 62, 1});
+        owner[61] = owner[62] = 1;
+        ds = gh_ds_from_arrays(62, labels.data(), edges.size() / 3, edges.data(), owner.data(), 2);
+        int rc = 0;
+        e = gh_engine_create(ds, 0, 1 << 20, &rc);
+        CHECK(e != nullptr && rc == GV_OK);
+        CHECK(gh_engine_resident_blocks(e) > 0);
+        CHECK(gh_engine_batch_config(e, 4, 1 << 20, 1 << 16, 0, 0) == GV_OK);
+    }
+    ~Served() {
+        gh_engine_free(e);
+        gh_ds_free(ds);
+    }
+    static std::string path(int k) {
+        std::string q;
+        for (int i = 0; i < k; ++i) q += "v " + std::to_string(i) + " 1\n";
+        for (int i = 0; i + 1 < k; ++i) q += "e " + std::to_string(i) + " " + std::to_string(i + 1) + " 1\n";
+        return q;
+    }
+    int serve(std::vector<int> ks, uint64_t budget) {   // all requests there at once
+        std::vector<std::string> text;
+        std::vector<const char*> q;
+        for (int k : ks) text.push_back(path(k));
+        for (auto& t : text) q.push_back(t.c_str());
+        std::vector<double> at(ks.size(), 0.0), latency(ks.size());
+        return gh_engine_serve(e, q.data(), at.data(), (uint32_t)ks.size(), 0, budget, latency.data(), nullptr, nullptr, 0, stats);
+    }
+};
+
+// The memory bound of a turn holds after a request whose estimate is out of
+// range as well.
+void bound_after_huge_estimate() {
+    fake::on_launch = pack_kernels;
+    Served s;
+    CHECK(s.serve({5, 5}, 1ull << 30) == GV_OK && s.stats[1] == 1);    // both in one turn
+    CHECK(s.serve({14, 5}, 1ull << 30) == GV_OK && s.stats[1] == 2);   // 2^64 - 1 and some MB
+    CHECK(s.serve({5, 14}, 1ull << 30) == GV_OK && s.stats[1] == 2);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -263,6 +312,7 @@ int main(int, char** argv) {
     else if (what == "packing_fails") packing_fails();
     else if (what == "no_host_memory") no_host_memory();
     else if (what == "counters_without_slot_engine") counters_without_slot_engine();
+    else if (what == "bound_after_huge_estimate") bound_after_huge_estimate();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
