@@ -130,9 +130,10 @@ static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
         out.latencyMs[r] = (atS - arrivalS[r]) * 1e3;
         ++finished;
     };
-    // a request on the plain path
-    auto direct = [&](size_t r) {
-        ++out.direct;
+    // a request on the plain path: one that the packed form does not take, or
+    // (refused) one of a turn that did not fit
+    auto direct = [&](size_t r, bool refused) {
+        ++(refused ? out.overflowed : out.direct);
         if (worker.enabled()) {
             worker.submit(r);
             return (int)GV_OK;
@@ -170,7 +171,7 @@ static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
             if (reqs[next].empty) {
                 finish(next, since(t0));
             } else if (!bm.residentTakes(reqs[next])) {
-                const int rc = direct(next);
+                const int rc = direct(next, false);
                 if (rc != GV_OK) return rc;
             } else {
                 // (estimates go up to 2^64 - 1: their sum may not)
@@ -203,7 +204,7 @@ static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
                                   nwords ? bits.data() : nullptr, nwords, nullptr);
         if (rc == GV_ERR_CAPACITY) {
             for (size_t r : now)
-                if ((rc = direct(r)) != GV_OK) return rc;
+                if ((rc = direct(r, true)) != GV_OK) return rc;
             continue;
         }
         if (rc != GV_OK) return rc;

@@ -301,6 +301,19 @@ void bound_after_huge_estimate() {
     CHECK(s.serve({5, 14}, 1ull << 30) == GV_OK && s.stats[1] == 2);
 }
 
+// Requests that a turn could not take are reported as overflowed, not as sent
+// straight to the plain path.
+void refused_turn_is_overflow() {
+    fake::on_launch = pack_kernels;
+    Served s;
+    fake::failed = false;
+    fake::fail_alloc = 3;   // after the side worker's context: the turn's first buffer
+    CHECK(s.serve({5, 5}, 1ull << 30) == GV_OK);
+    fake::fail_alloc = -1;
+    CHECK(fake::failed && s.stats[3] == 2 && s.stats[4] == 0);
+    CHECK(s.serve({5, 5}, 1ull << 30) == GV_OK && s.stats[3] == 0 && s.stats[4] == 0);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -313,6 +326,7 @@ int main(int, char** argv) {
     else if (what == "no_host_memory") no_host_memory();
     else if (what == "counters_without_slot_engine") counters_without_slot_engine();
     else if (what == "bound_after_huge_estimate") bound_after_huge_estimate();
+    else if (what == "refused_turn_is_overflow") refused_turn_is_overflow();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
