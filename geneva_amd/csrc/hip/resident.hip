@@ -1470,7 +1470,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         }
         const uint32_t fixed = R->img_bytes + 16 * nops + 4 * p.nterms * R->gw + 16 + kRCtlBytes;
         const uint32_t each = rwave_bytes(p.lvl_bytes, p.lmax);
-        uint32_t waves = kRSmallWaves;
+        uint32_t waves = fixed < kRLdsMost ? std::min(kRSmallWaves, (kRLdsMost - fixed) / each) : 0;
         if (!small) {
             // the split of a CU's LDS that holds the most waves, in two
             // workgroups or more: one alone idles at each change of block

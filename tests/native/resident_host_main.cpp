@@ -314,6 +314,57 @@ void refused_turn_is_overflow() {
     CHECK(s.serve({5, 5}, 1ull << 30) == GV_OK && s.stats[3] == 0 && s.stats[4] == 0);
 }
 
+// A query of 16 vertices whose levels take 27 KiB a wave, on a database with a
+// graph of nearly 64 KiB: with three waves it fits LDS.
+void wide_levels_beside_a_large_graph() {
+    fake::on_launch = pack_kernels;
+    // a path of n vertices and a pair, one label, as a partition block
+    const uint32_t n = 4600, nv = n + 2;
+    std::vector<uint32_t> labels(nv + 1, 1), owner(nv + 1, 0), at(1, 0), list;
+    labels[0] = nv;
+    owner[n + 1] = owner[n + 2] = 1;
+    for (uint32_t v = 1; v <= nv; ++v) {
+        if (v != 1 && v != n + 1) list.push_back(v - 1);
+        if (v != n && v != nv) list.push_back(v + 1);
+        at.push_back((uint32_t)list.size());
+    }
+    std::vector<uint32_t> block{0, nv, 1, 0, 4 + nv + 1, /*sources*/ 1, 0, nv, 0};
+    block.insert(block.end(), at.begin(), at.end());
+    // a list of up to 130 neighbours has no skip index before it
+    block.insert(block.end(), list.begin(), list.end());
+    block[0] = (uint32_t)block.size();
+    const uint32_t* blocks[] = {block.data()};
+    const uint32_t edge_label = 1;
+    gv_ctx_t c = nullptr;
+    gv_graph_t g = nullptr;
+    CHECK(gv_ctx_create(0, &c) == GV_OK);
+    CHECK(gv_graph_create(c, labels.data(), 1, blocks, &edge_label, &g) == GV_OK);
+    CHECK(gv_graph_set_owner(g, owner.data(), 2) == GV_OK);
+    CHECK(packed_bytes(g) > 64000);
+    gv_query_t q{};
+    q.k = 16;
+    for (uint32_t w = 1; w < q.k; ++w) {
+        gv_step_t& s = q.step[w];
+        s.col = w;
+        s.nback = 1;   // column 0
+        s.restrict_col = GV_NONE;
+    }
+    // columns 0 to 9 are read by the last two steps, so every table keeps them
+    q.step[15].nback = 3;
+    q.step[15].back_col[1] = 1;
+    q.step[15].back_col[2] = 2;
+    q.step[15].ncoll = q.step[14].ncoll = 4;
+    for (uint32_t i = 0; i < 4; ++i) {
+        q.step[15].coll_col[i] = 3 + i;
+        q.step[14].coll_col[i] = 6 + i;
+    }
+    const gv_query_t* qs[] = {&q};
+    uint64_t count = 0, bytes = 0;
+    CHECK(gv_resident_mine(c, g, 1, qs, nullptr, &count, &bytes, nullptr, 0, nullptr) == GV_OK);
+    gv_graph_destroy(g);
+    gv_ctx_destroy(c);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -327,6 +378,7 @@ int main(int, char** argv) {
     else if (what == "counters_without_slot_engine") counters_without_slot_engine();
     else if (what == "bound_after_huge_estimate") bound_after_huge_estimate();
     else if (what == "refused_turn_is_overflow") refused_turn_is_overflow();
+    else if (what == "wide_levels_beside_a_large_graph") wide_levels_beside_a_large_graph();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
