@@ -108,9 +108,10 @@ private:
 // requests that have arrived, as many as the engine has slots and the memory
 // bound admits, and mines them in one call, in which they share their common
 // steps.  A request the packed form does not take goes to the plain path.
-// A lone request waits kCompanyS for another: a launch costs both about
-// 30 us, and requests that arrive together are then one iteration, which the
-// memory bound splits.
+// Requests that arrive within kCompanyS of each other are one iteration, which
+// the memory bound splits: a lone request that came so soon after the one
+// before it waits that long for another.  Others do not wait (1,000 requests a
+// second on 20,000 graphs: p50 48 us, with every lone request waiting 68).
 constexpr double kCompanyS = 20e-6;
 static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
                          const std::vector<double>& arrivalS, uint64_t memBudget,
@@ -162,8 +163,8 @@ static int serveResident(BatchMiner& bm, const std::vector<CompiledQuery>& reqs,
         uint64_t inUse = 0;
         for (; next < n && now.size() < slots; ++next) {
             if (arrivalS[next] > since(t0)) {
-                // nothing more has arrived; a lone, fresh request waits
-                if (now.size() != 1) break;
+                // nothing more has arrived
+                if (now.size() != 1 || now[0] == 0 || arrivalS[now[0]] - arrivalS[now[0] - 1] >= kCompanyS) break;
                 while (arrivalS[next] > since(t0) && since(t0) < arrivalS[now[0]] + kCompanyS) {
                 }
                 if (arrivalS[next] > since(t0)) break;

@@ -4,6 +4,7 @@
 #include "geneva_hip.h"
 #include "geneva_host.h"
 
+#include <algorithm>
 #include <new>
 
 // host allocations until one throws (-1: none does)
@@ -281,12 +282,15 @@ struct Served {
         for (int i = 0; i + 1 < k; ++i) q += "e " + std::to_string(i) + " " + std::to_string(i + 1) + " 1\n";
         return q;
     }
-    int serve(std::vector<int> ks, uint64_t budget) {   // all requests there at once
+    std::vector<double> latency;
+    int serve(std::vector<int> ks, uint64_t budget, double apart = 0.0) {   // requests this far apart
         std::vector<std::string> text;
         std::vector<const char*> q;
         for (int k : ks) text.push_back(path(k));
         for (auto& t : text) q.push_back(t.c_str());
-        std::vector<double> at(ks.size(), 0.0), latency(ks.size());
+        std::vector<double> at;
+        for (size_t i = 0; i < ks.size(); ++i) at.push_back(apart * (double)i);
+        latency.assign(ks.size(), 0.0);
         return gh_engine_serve(e, q.data(), at.data(), (uint32_t)ks.size(), 0, budget, latency.data(), nullptr, nullptr, 0, stats);
     }
 };
@@ -365,6 +369,18 @@ void wide_levels_beside_a_large_graph() {
     gv_ctx_destroy(c);
 }
 
+// A request that comes long after the one before it is mined at once, also
+// with others to come.
+void lone_request_does_not_wait() {
+    fake::on_launch = pack_kernels;
+    Served s;
+    CHECK(s.serve(std::vector<int>(100, 5), 1ull << 30, 0.5e-3) == GV_OK);
+    double least = 1e9;
+    for (size_t i = 0; i + 1 < s.latency.size(); ++i) least = std::min(least, s.latency[i]);
+    std::printf("least latency %.1f us\n", least * 1e3);
+    CHECK(least < 20e-3);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -379,6 +395,7 @@ int main(int, char** argv) {
     else if (what == "bound_after_huge_estimate") bound_after_huge_estimate();
     else if (what == "refused_turn_is_overflow") refused_turn_is_overflow();
     else if (what == "wide_levels_beside_a_large_graph") wide_levels_beside_a_large_graph();
+    else if (what == "lone_request_does_not_wait") lone_request_does_not_wait();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;
