@@ -27,6 +27,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+LDS_PEAK_GBS = 256 * 128 * 2.4   # CUs x bytes a clock x GHz
 
 
 def log(*a):
@@ -338,12 +339,12 @@ def section_w3(args):
     b_total = sum(r.alg_bytes for r in acct_res)
     if launches:
         achieved = b_ran / (dev_ms / 1e3) / 1e9 if dev_ms > 0 else 0.0
-        roofline = {"bound": "lds", "kernel": "k_resident", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                    "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "launches": launches,
+        roofline = {"bound": "lds", "kernel": "k_resident", "achieved": round(achieved, 2), "peak": LDS_PEAK_GBS,
+                    "unit": "GB/s", "frac": round(achieved / LDS_PEAK_GBS, 4), "traffic": None, "launches": launches,
                     "avg_launch_ms": round(dev_ms / launches, 4), "total_ms": round(dev_ms, 3),
                     "b_bytes_per_launch": b_ran // launches, "b_bytes_of_queries": b_total,
                     "b_charged": "B of every step run, steps shared between queries once; the kernel reads it out "
-                                 "of LDS, so HBM's rate is a scale here and no limit"}
+                                 "of LDS"}
         kern = {"k_resident": {"launches": launches, "ms": round(dev_ms, 3)}}
     else:
         roofline, kern = slots_roofline(eng, qs)

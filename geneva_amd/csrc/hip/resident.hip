@@ -1015,7 +1015,7 @@ constexpr uint64_t kRTailBytes = 4 * kRDoneStep * (1 + kRLines);
 
 // A context's buffers of gv_resident_mine, kept between calls (grow only).
 struct ResWork {
-    char* d_prog = nullptr;               // operations, leaf descriptors, roots
+    char* d_prog = nullptr;               // the program (RProg::image) and the tasks
     char* h_prog = nullptr;               // pinned
     uint64_t prog_cap = 0;
     // kRLines copies of 2 kRMaxOps words, the counters (kTail...), zero between
@@ -1042,7 +1042,7 @@ void res_work_free(gv_ctx* c) {
 namespace {
 
 // The operations of a launch: tables and the steps on them, added query by
-// query, then laid out as ROp / RLeaf.
+// query, then laid out as ROp, RMore and RLeafStep.
 struct RProg {
     struct Op {
         uint32_t kind, table, child = kNone, term = kNone;   // child: table

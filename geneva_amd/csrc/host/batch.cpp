@@ -159,17 +159,18 @@ int BatchMiner::runResident(const std::vector<CompiledQuery>& qs, const std::vec
         bits[i] = out[order[i]].graphBits.data();
     }
     gv_mark(ctx_, 2);
+    gv_resident_stats_t did{};
     int rc = gv_resident_mine(ctx_, g_, (uint32_t)n, q.data(), lv.data(), count.data(), bytes.data(),
-                              nwords_ ? bits.data() : nullptr, nwords_, &res_);
+                              nwords_ ? bits.data() : nullptr, nwords_, &did);
     if (rc != GV_OK) return rc;
     gv_mark(ctx_, 3);
     float ms = 0;
     gv_elapsed_ms(ctx_, 2, 3, &ms);
     st.deviceMs = ms;
     st.batched = n;
-    st.graphLaunches += res_.launches;
-    resShared_ += res_.shared_queries;
-    resFused_ += res_.fused_rows;
+    st.graphLaunches += did.launches;
+    resShared_ += did.shared_queries;
+    resFused_ += did.fused_rows;
     for (size_t i = 0; i < n; ++i) {
         out[order[i]].count = count[i];
         out[order[i]].algBytes = bytes[i];
@@ -218,7 +219,6 @@ int BatchMiner::run(const std::vector<CompiledQuery>& qs, std::vector<MineResult
     std::stable_sort(order.begin(), order.end(),
                      [&](size_t a, size_t b) { return startKey(a) < startKey(b); });
     BatchStats local;
-    res_ = gv_resident_stats_t{};
     if (resident()) {
         // the packed form takes what it can, the slot engine the others
         std::vector<size_t> packed, rest;

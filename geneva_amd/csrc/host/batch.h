@@ -76,8 +76,6 @@ public:
     int fusedRows(uint64_t* rows);
     // The slot engine runs every query from now on (autotuning).
     void useSlots(bool on) { slotsOnly_ = on; }
-    // What the last run out of a packed database did (all zero otherwise).
-    const gv_resident_stats_t& residentStats() const { return res_; }
 
     // Mine every query; results in input order.  Queries with a plan error
     // get status GV_ERR_ARG; overflowing ones are re-run on the plain path.
@@ -114,7 +112,6 @@ private:
     BatchOptions opt_;
     bool share_ = true, fuse_ = true, pairStart_ = true, profile_ = false, slotsOnly_ = false;
     uint64_t resShared_ = 0, resFused_ = 0;
-    gv_resident_stats_t res_{};
     gv_batch_t b_ = nullptr;
     uint32_t nwords_ = 0;
     uint64_t rowCap_ = 0;

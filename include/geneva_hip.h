@@ -391,7 +391,7 @@ int gv_resident_info(gv_graph_t g, uint32_t* blocks, uint64_t* bytes);
 int gv_resident_ready(gv_ctx_t ctx, gv_graph_t g);
 
 typedef struct {
-    uint64_t launches;        /* mining launches */
+    uint64_t launches;        /* mining launches (several where the work sits in few blocks) */
     uint64_t shared_queries;  /* queries that share their first steps with an earlier one */
     uint64_t fused_rows;      /* rows read again for another step on the same table */
     uint64_t rows;            /* rows read, shared ones once */
