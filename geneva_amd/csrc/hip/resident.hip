@@ -148,7 +148,11 @@ constexpr uint32_t kRLeastRows = 16;             // start rows of a share
 constexpr uint32_t kRLdsMost = 160u << 10;       // LDS of a CU
 constexpr uint32_t kRSmallWaves = 4, kRWaves = 8;   // waves of a workgroup, at most
 constexpr uint32_t kRGive = 16;                  // rows of a table worth sharing; 4 or 48: within 2%
-constexpr uint64_t kRAsideBytes = 4u << 20;      // tables set aside by one launch, at most
+// Room for the tables that one launch sets aside: at first (a call on a new
+// context pays for the allocation: with 4 MiB 920 us instead of 310), and
+// after a call that set aside more (131 queries on 6,000 graphs: with 512 KiB
+// 2.95 ms, with 4 MiB 1.55).
+constexpr uint64_t kRAsideFirst = 512u << 10, kRAsideMost = 4u << 20;
 // A wave sets tables aside once it has worked through kRSpare batches of 64
 // rows or 64 candidates in a block (about 80 us alone), while a quarter of the
 // workgroups that the chip holds or fewer are at work; it looks again every
@@ -1018,9 +1022,11 @@ struct ResWork {
     char* d_prog = nullptr;               // the program (RProg::image) and the tasks
     char* h_prog = nullptr;               // pinned
     uint64_t prog_cap = 0;
-    // kRLines copies of 2 kRMaxOps words, the counters (kTail...), zero between
-    // calls; then twice kRAsideBytes of tables set aside
+    // kRLines copies of 2 kRMaxOps words and the counters (kTail...), zero
+    // between calls
     unsigned long long* d_acc = nullptr;
+    uint32_t* d_aside = nullptr;          // tables set aside: twice aside_bytes
+    uint64_t aside_bytes = 0, aside_want = kRAsideFirst;
     unsigned long long* h_acc = nullptr;  // pinned: 2 kRMaxOps words and the number set aside
     uint32_t* d_bits = nullptr;           // zero between calls
     uint32_t* h_bits = nullptr;           // pinned
@@ -1031,7 +1037,7 @@ struct ResWork {
 void res_work_free(gv_ctx* c) {
     ResWork* w = c->resw;
     if (!w) return;
-    for (void* p : {(void*)w->d_prog, (void*)w->d_acc, (void*)w->d_bits})
+    for (void* p : {(void*)w->d_prog, (void*)w->d_acc, (void*)w->d_aside, (void*)w->d_bits})
         if (p) (void)hipFree(p);
     for (void* p : {(void*)w->h_prog, (void*)w->h_acc, (void*)w->h_bits})
         if (p) (void)hipHostFree(p);
@@ -1351,7 +1357,7 @@ int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
     // (each of the two on its own: a call that found memory for one of them
     // only leaves that one for the next)
     if (!w->d_acc) {
-        if (hipMalloc(&w->d_acc, kRAccBytes + kRTailBytes + 2 * kRAsideBytes) != hipSuccess) {
+        if (hipMalloc(&w->d_acc, kRAccBytes + kRTailBytes) != hipSuccess) {
             w->d_acc = nullptr;
             return GV_ERR_NOMEM;
         }
@@ -1360,6 +1366,20 @@ int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
     if (!w->h_acc && hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps + 16, hipHostMallocCoherent) != hipSuccess) {
         w->h_acc = nullptr;
         return GV_ERR_NOMEM;
+    }
+    if (w->aside_want > w->aside_bytes) {
+        uint32_t* room = nullptr;
+        if (hipMalloc(&room, 2 * w->aside_want) == hipSuccess) {
+            HIPCHK(hipStreamSynchronize(c->stream));
+            if (w->d_aside) HIPCHK(hipFree(w->d_aside));
+            w->d_aside = room;
+            w->aside_bytes = w->aside_want;
+        } else if (w->d_aside) {
+            (void)hipGetLastError();   // what there is does as well
+            w->aside_want = w->aside_bytes;
+        } else {
+            return GV_ERR_NOMEM;
+        }
     }
     if (prog > w->prog_cap) {
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -1451,13 +1471,13 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         a.nwords = nwords;
         a.acc = w->d_acc;
         uint32_t* const tail = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(w->d_acc) + kRAccBytes);
-        uint32_t* const aside[2] = {tail + kRTailBytes / 4, tail + (kRTailBytes + kRAsideBytes) / 4};
+        uint32_t* const aside[2] = {w->d_aside, w->d_aside + w->aside_bytes / 4};
         uint32_t* const left = reinterpret_cast<uint32_t*>(w->h_acc + 2 * kRMaxOps);
         a.next = tail + kTailNext;
         a.done = tail + kTailDone;
         a.nwork = R->nblk;
         a.item_words = kRAside + 64 * p.most_cols;
-        a.aside_cap = (uint32_t)(kRAsideBytes / 4 / a.item_words);
+        a.aside_cap = (uint32_t)(w->aside_bytes / 4 / a.item_words);
         a.bits = bits ? w->d_bits : nullptr;
         if (small) {
             p.image(reinterpret_cast<char*>(a.prog));
@@ -1512,6 +1532,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
             HIPCHK(hipStreamSynchronize(c->stream));
             st.launches += 1;
             if (*left == 0) break;
+            if (*left > a.aside_cap) w->aside_want = kRAsideMost;
             // the tables that were set aside, over the whole chip
             a.items = a.aside;
             a.nwork = std::min<uint32_t>(*left, a.aside_cap);

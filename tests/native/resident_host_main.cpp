@@ -381,6 +381,35 @@ void lone_request_does_not_wait() {
     CHECK(least < 20e-3);
 }
 
+// A call that sets aside more than there is room for gets more room in the
+// next one, and does without where there is no memory for it.
+uint32_t set_aside = 0;   // what the next launch sets aside
+hipError_t sets_aside(const std::string& name, void** args) {
+    if (name.find("k_resident_out") != std::string::npos) {
+        **(uint32_t**)args[9] = set_aside;
+        set_aside = 0;
+    }
+    return hipSuccess;
+}
+void room_for_tables_set_aside() {
+    fake::on_launch = sets_aside;
+    fake::sticky = true;
+    Db db;
+    CHECK(gv_graph_set_owner(db.g, kOwner, 2) == GV_OK);
+    CHECK(db.mine() == GV_OK);
+    int held = fake::allocations;
+    set_aside = 5;
+    CHECK(db.mine() == GV_OK && db.mine() == GV_OK && fake::allocations == held);
+    set_aside = 1u << 20;
+    CHECK(db.mine() == GV_OK && fake::allocations == held);
+    fake::fail_alloc = 0;
+    CHECK(db.mine() == GV_OK && fake::allocations == held && fake::last == hipSuccess);
+    set_aside = 1u << 20;
+    CHECK(db.mine() == GV_OK && db.mine() == GV_OK && fake::allocations == held + 1);
+    set_aside = 1u << 20;
+    CHECK(db.mine() == GV_OK && db.mine() == GV_OK && fake::allocations == held + 1);
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -396,6 +425,7 @@ int main(int, char** argv) {
     else if (what == "refused_turn_is_overflow") refused_turn_is_overflow();
     else if (what == "wide_levels_beside_a_large_graph") wide_levels_beside_a_large_graph();
     else if (what == "lone_request_does_not_wait") lone_request_does_not_wait();
+    else if (what == "room_for_tables_set_aside") room_for_tables_set_aside();
     else return 2;
     std::printf("%s: %d wrong\n", what.c_str(), fails);
     return fails ? 1 : 0;

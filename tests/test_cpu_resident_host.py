@@ -31,7 +31,7 @@ def exe(tmp_path_factory):
                                   "owners_on_their_device", "packing_fails", "no_host_memory",
                                   "counters_without_slot_engine", "bound_after_huge_estimate",
                                   "refused_turn_is_overflow", "wide_levels_beside_a_large_graph",
-                                  "lone_request_does_not_wait"])
+                                  "lone_request_does_not_wait", "room_for_tables_set_aside"])
 def test_resident_host(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
