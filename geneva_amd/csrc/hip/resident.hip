@@ -18,13 +18,14 @@
 // What bounds it: a wave's chain of dependent LDS reads and scalar
 // instructions for each batch of 64 rows and each 64 of their candidates, so
 // the waves a CU holds (its LDS) and how evenly they are kept busy.  Measured
-// on MI355X, calls on three seeds each, before = the table engines (a launch
+// on MI355X, means of four databases each, before = the table engines (a launch
 // or more per step of a query, tables in HBM):
-//   10 queries on 1,000 small graphs, one by one      939 ->  380 us
-//   24 queries on 20,000 graphs, one by one          4532 -> 1957 us
-//   131 queries on 17,321 graphs, one call           3.08 -> 1.77 ms
-//   256 queries on 100,000 graphs, one call          16.9 -> 9.24 ms
-// The split of the work that gives these: workgroups take blocks as they
+//   10 queries on 1,000 small graphs, one by one      849 ->  375 us
+//   24 queries on 20,000 graphs, one by one          4714 -> 1890 us
+//   131 queries on 17,321 graphs, one call           3.33 -> 1.65 ms
+//   256 queries on 100,000 graphs, one call          18.8 -> 9.79 ms
+// The split of the work that gives these (figures below are of earlier states,
+// each beside its own reference): workgroups take blocks as they
 // become free (with every gridDim-th block 3.05 and 11.1 ms), their waves take
 // tasks of a block, and a wave without a task gets half of the next table that
 // another one makes: one start vertex can hold most of a block's work (without
@@ -1027,7 +1028,7 @@ struct ResWork {
     unsigned long long* d_acc = nullptr;
     uint32_t* d_aside = nullptr;          // tables set aside: twice aside_bytes
     uint64_t aside_bytes = 0, aside_want = kRAsideFirst;
-    unsigned long long* h_acc = nullptr;  // pinned: 2 kRMaxOps words and the number set aside
+    unsigned long long* h_acc = nullptr;  // pinned: the number set aside, then 2 kRMaxOps words
     uint32_t* d_bits = nullptr;           // zero between calls
     uint32_t* h_bits = nullptr;           // pinned
     uint64_t bits_cap = 0;
@@ -1363,9 +1364,12 @@ int res_buffers(gv_ctx* c, uint64_t prog, uint64_t bits) {
         }
         w->dirty = true;
     }
-    if (!w->h_acc && hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps + 16, hipHostMallocCoherent) != hipSuccess) {
-        w->h_acc = nullptr;
-        return GV_ERR_NOMEM;
+    if (!w->h_acc) {
+        if (hipHostMalloc((void**)&w->h_acc, 16 * kRMaxOps + 16, hipHostMallocCoherent) != hipSuccess) {
+            w->h_acc = nullptr;
+            return GV_ERR_NOMEM;
+        }
+        *w->h_acc = 0;
     }
     if (w->aside_want > w->aside_bytes) {
         uint32_t* room = nullptr;
@@ -1472,7 +1476,8 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         a.acc = w->d_acc;
         uint32_t* const tail = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(w->d_acc) + kRAccBytes);
         uint32_t* const aside[2] = {w->d_aside, w->d_aside + w->aside_bytes / 4};
-        uint32_t* const left = reinterpret_cast<uint32_t*>(w->h_acc + 2 * kRMaxOps);
+        unsigned long long* const sums = w->h_acc + 1;
+        uint32_t* const left = reinterpret_cast<uint32_t*>(w->h_acc);
         a.next = tail + kTailNext;
         a.done = tail + kTailDone;
         a.nwork = R->nblk;
@@ -1516,7 +1521,6 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         for (uint32_t turn = 0;; ++turn) {
             a.aside = aside[turn & 1];
             a.naside = tail + kTailAside + (turn & 1);
-            *left = 0;
             {
                 ProfScope ps(c, kKindResident);
                 const uint32_t grid = std::min<uint32_t>(a.nwork, per_cu * c->num_cu);
@@ -1526,7 +1530,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
                 HIPCHK(hipGetLastError());
             }
             hipLaunchKernelGGL(k_resident_out, dim3(grid_for(std::max<uint64_t>(nb, 2 * nops), 256, 512)), dim3(256), 0,
-                               c->stream, w->d_acc, 2 * nops, w->h_acc, a.next, w->d_bits, nb, w->h_bits,
+                               c->stream, w->d_acc, 2 * nops, sums, a.next, w->d_bits, nb, w->h_bits,
                                tail + kTailAside, turn & 1, left, a.done);
             HIPCHK(hipGetLastError());
             HIPCHK(hipStreamSynchronize(c->stream));
@@ -1543,8 +1547,8 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
         for (uint32_t x = 0; x < nops; ++x) {
             const RProg::Op& o = p.ops[x];
             const RProg::Table& t = p.tables[o.table];
-            const uint64_t lists = w->h_acc[2 * x], found = w->h_acc[2 * x + 1];
-            const uint64_t rows = t.from == kNone ? g->lvoff[t.label0 + 1] - g->lvoff[t.label0] : w->h_acc[2 * t.from + 1];
+            const uint64_t lists = sums[2 * x], found = sums[2 * x + 1];
+            const uint64_t rows = t.from == kNone ? g->lvoff[t.label0 + 1] - g->lvoff[t.label0] : sums[2 * t.from + 1];
             by[x] = o.kind == kOpLeaves ? lists
                                         : rows * (4ull * t.width + 8ull * o.st.nback) + 4 * lists +
                                               (o.kind == kOpExtend ? 4ull * (t.width + 1) * found : 0ull);
@@ -1556,7 +1560,7 @@ int resident_mine(gv_ctx_t c, gv_graph_t g, uint32_t n, const gv_query_t* const*
             const std::vector<uint32_t>& path = paths[i - i0];
             uint64_t b = 0;
             for (uint32_t x : path) b += by[x];
-            counts[i] = w->h_acc[2 * path.back() + 1];
+            counts[i] = sums[2 * path.back() + 1];
             alg_bytes[i] = b;
             if (bits && bits[i]) memcpy(bits[i], w->h_bits + (uint64_t)p.ops[path.back()].term * nwords, 4ull * nwords);
         }
