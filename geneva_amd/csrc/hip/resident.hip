@@ -681,16 +681,22 @@ __global__ __launch_bounds__(1024) void k_resident(RArgs a) {
         __syncthreads();
         const uint32_t wnext = gridDim.x + (counter ? uni(ld32(o_ctl + kCtlNext)) : uni(wv));
         if (a.bits) {
-            // (read again: they are not worth registers while the block is mined)
+            // (a batch reads them again: they are not worth registers while the
+            // block is mined; one small query would wait for them)
             const GV_CONST RArgs& a = rargs();
-            const RBlk& blk = a.blk[kAside ? a.items[(uint64_t)uni(wv) * a.item_words] : uni(wv)];
-            for (uint32_t i = threadIdx.x; i < a.nterms * blk.gwords; i += blockDim.x) {
-                const uint32_t term = i / blk.gwords, x = i - term * blk.gwords;
+            uint32_t gwords = blk.gwords, graph0 = blk.graph0;
+            if constexpr (!kSmall) {
+                const RBlk& again = a.blk[kAside ? a.items[(uint64_t)uni(wv) * a.item_words] : uni(wv)];
+                gwords = again.gwords;
+                graph0 = again.graph0;
+            }
+            for (uint32_t i = threadIdx.x; i < a.nterms * gwords; i += blockDim.x) {
+                const uint32_t term = i / gwords, x = i - term * gwords;
                 const uint32_t o = o_bits + 4 * (term * a.gw + x);
                 const uint32_t m = ld32(o);
                 if (m) {
                     st32(o, 0);
-                    atomicOr(&a.bits[(uint64_t)term * a.nwords + (blk.graph0 >> 5) + x], m);
+                    atomicOr(&a.bits[(uint64_t)term * a.nwords + (graph0 >> 5) + x], m);
                 }
             }
         }
